@@ -41,6 +41,7 @@ SPM_INT_WALK_AUTO = 0
 SPM_INT_WALK_INT32 = 1
 SPM_INT_WALK_FP64 = 2
 SPM_INT_WALK_SPARSE = 3
+SPM_INT_WALK_PRUNED = 4
 
 SPM_DECOMP_DM = 1
 SPM_DECOMP_COMPONENTS = 2

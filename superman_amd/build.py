@@ -47,6 +47,8 @@ SOURCES = [  # the longest compiles first, so that the job pool starts them earl
     ("dense_f64.hip", []),
     ("int_sparse.hip", []),
     ("int_small.hip", []),
+    ("int_prune.hip", []),
+    ("prune.cpp", []),
     ("batch_engine.cpp", []),
     ("decompose.cpp", []),
     ("codegen.cpp", []),

@@ -35,7 +35,7 @@ std::mutex g_mu;
 struct OccEntry {
     int device;
     const void* kern;
-    int block;
+    int block, lds;
     int bpc;
 };
 std::vector<OccEntry> g_occ;
@@ -61,20 +61,20 @@ int device_cus(int device, int* cus)
     return SPM_OK;
 }
 
-int blocks_per_cu(int device, const void* kern, int block, int* bpc)
+int blocks_per_cu(int device, const void* kern, int block, int* bpc, int lds_bytes)
 {
     {
         std::lock_guard<std::mutex> lk(g_mu);
         for (const auto& e : g_occ)
-            if (e.device == device && e.kern == kern && e.block == block) {
+            if (e.device == device && e.kern == kern && e.block == block && e.lds == lds_bytes) {
                 *bpc = e.bpc;
                 return SPM_OK;
             }
     }
     int v = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, kern, block, 0) != hipSuccess || v <= 0) return SPM_EHIP;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, kern, block, lds_bytes) != hipSuccess || v <= 0) return SPM_EHIP;
     std::lock_guard<std::mutex> lk(g_mu);
-    g_occ.push_back({device, kern, block, v});
+    g_occ.push_back({device, kern, block, lds_bytes, v});
     *bpc = v;
     return SPM_OK;
 }
@@ -175,6 +175,14 @@ struct spm_plan {
     double* d_out = nullptr;
     double* h_out = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    int block = kDenseBlock;
+    int lds_bytes = 0;       // integer kind, pruned walk: dynamic LDS
+    unsigned int* d_counter = nullptr;  // its counters, a set per launch (0 between runs)
+    unsigned long long* d_list[2] = {nullptr, nullptr};
+    unsigned int list_cap = 0;          // prefixes per list segment
+    int first_group = 0;                // PrunePlan::first_group
+    const void* kern2 = nullptr;        // the walk over the listed nodes
+    int grid2 = 0;
     std::string kname;
     hipFunction_t fn = nullptr;  // generated kernel (kind 4), owned by the module cache
     uint64_t hash = 0;
@@ -189,6 +197,9 @@ static void plan_free(spm_plan* p)
     if (p->d_M) (void)hipFree(p->d_M);
     if (p->d_x0) (void)hipFree(p->d_x0);
     if (p->d_partial) (void)hipFree(p->d_partial);
+    if (p->d_counter) (void)hipFree(p->d_counter);
+    for (unsigned long long* l : p->d_list)
+        if (l) (void)hipFree(l);
     if (p->d_out) (void)hipFree(p->d_out);
     if (p->h_out) (void)hipHostFree(p->h_out);
     if (p->ev0) (void)hipEventDestroy(p->ev0);
@@ -311,15 +322,87 @@ static int int_prepare(const int64_t* a, int n, std::vector<int>& y0, double* lo
     return spm::int_prepare(a, n, y0.data(), log2_bound, w);
 }
 
+// Exact integer plans over the subsets with no zero row (kind 3).
+static int make_prune_plan(const PrunePlan& pr, int n, double log2_bound, int halved, int device, spm_plan** out)
+{
+    int cus = 0;
+    int st = device_cus(device, &cus);
+    if (st != SPM_OK) return st;
+    DeviceGuard guard(device);
+    if (!guard.ok()) return SPM_EHIP;
+    spm_plan* p = new spm_plan;
+    p->kind = 3;
+    p->n = n;
+    p->precision = -1;
+    p->device = device;
+    p->log2_bound = log2_bound;
+    p->halved = halved;
+    p->rec = 2;
+    p->comps = 0;
+    p->block = kPruneBlock;
+    p->lds_bytes = pr.lds_bytes;
+    p->tasks = pr.prefixes;
+    p->first_group = pr.first_group;
+    p->kern = int_prune_kernel_ptr(pr.field_bytes, pr.dwords, false);
+    p->kern2 = int_prune_kernel_ptr(pr.field_bytes, pr.dwords, true);
+    int bpc = 0, bpc2 = 0;
+    st = p->kern && p->kern2 ? blocks_per_cu(device, p->kern, p->block, &bpc, p->lds_bytes) : SPM_EINVAL;
+    if (st == SPM_OK) st = blocks_per_cu(device, p->kern2, p->block, &bpc2, p->lds_bytes);
+    if (st != SPM_OK) {
+        plan_free(p);
+        return st;
+    }
+    const uint64_t waves = p->block / kWaveLanes;
+    p->grid = bpc * cus;
+    p->grid2 = bpc2 * cus;
+    if (p->first_group == 2) {
+        p->grid = 0;
+        p->grid2 = (int)std::min<uint64_t>(p->grid2, (p->tasks + waves - 1) / waves);
+    } else {
+        // The estimate takes the rows as independent; the survivors of
+        // uniform patterns run up to ~10x it.  At most 2^(n-13) nodes exist,
+        // and prefixes past 2^22 (2 x 42 MB) are walked where they are found.
+        const double cap = std::min(64.0 * std::max(pr.nodes, pr.upper), std::ldexp(1.0, std::min(22, n - 13)));
+        p->list_cap = (unsigned)std::max(512.0, std::ceil(cap * 1.25 / kPruneSets));
+        for (unsigned long long*& l : p->d_list)
+            if (hipMalloc(&l, sizeof(unsigned long long) * p->list_cap * kPruneSets) != hipSuccess) {
+                (void)hipGetLastError();
+                l = nullptr;
+                plan_free(p);
+                return SPM_ENOMEM;
+            }
+    }
+    char kn[96];
+    std::snprintf(kn, sizeof kn, "int_prune_kernel<%d, %d>", pr.field_bytes, pr.dwords);
+    p->kname = kn;
+    SPM_TRY(hipMalloc(&p->d_M, sizeof(int) * pr.blob.size()));
+    SPM_TRY(hipMemcpy(p->d_M, pr.blob.data(), sizeof(int) * pr.blob.size(), hipMemcpyHostToDevice));
+    const int records = p->grid * (p->first_group - 2) + p->grid2;  // a record per block and launch
+    const size_t counters = sizeof(unsigned int) * kPruneSets * kPruneCounterStride * p->first_group;
+    SPM_TRY(hipMalloc(&p->d_counter, counters));
+    SPM_TRY(hipMemset(p->d_counter, 0, counters));
+    SPM_TRY(hipMalloc(&p->d_partial, sizeof(unsigned long long) * 2 * records));
+    p->partial_cap = records;
+    SPM_TRY(hipMalloc(&p->d_out, sizeof(double) * 6));
+    SPM_TRY(hipHostMalloc(&p->h_out, sizeof(double) * 6, hipHostMallocDefault));
+    SPM_TRY(hipEventCreate(&p->ev0));
+    SPM_TRY(hipEventCreate(&p->ev1));
+    *out = p;
+    return SPM_OK;
+}
+
 // Exact integer plans (kind 3): y = 2x in int32, T mod 2^128.
-// walk: SPM_INT_WALK_AUTO picks the FP64 walk when every absolute row sum is
-// below 2^int_small_bits(n) (int_small_ok), else the int32 walk.
+// walk: SPM_INT_WALK_AUTO picks the walk over the subsets with no zero row
+// where its estimate is the lowest (prune_preferred), else the
+// compressed-column walk where that one's is (int_sparse_preferred), else the
+// FP64 walk when every absolute row sum is below 2^int_small_bits(n)
+// (int_small_ok), else the int32 walk.
 static int make_int_plan(const int64_t* a, int n, int walk, int device, spm_plan** out)
 {
     if (!out) return SPM_EINVAL;
     *out = nullptr;
     if (walk != SPM_INT_WALK_AUTO && walk != SPM_INT_WALK_INT32 && walk != SPM_INT_WALK_FP64 &&
-        walk != SPM_INT_WALK_SPARSE)
+        walk != SPM_INT_WALK_SPARSE && walk != SPM_INT_WALK_PRUNED)
         return SPM_EINVAL;
     if (!a || n < 1 || n > kMaxN) return SPM_EINVAL;
     // rows with even sums carried halved (int_row_weights); the column sort
@@ -332,6 +415,16 @@ static int make_int_plan(const int64_t* a, int n, int walk, int device, spm_plan
     if (rc != SPM_OK) return rc;
     const bool small = int_small_ok(a, n);
     if (walk == SPM_INT_WALK_FP64 && !small) return SPM_ERANGE;
+    if (walk == SPM_INT_WALK_PRUNED || (walk == SPM_INT_WALK_AUTO && n >= kPruneAutoN)) {
+        PrunePlan pr;
+        const bool ok = prune_plan(a, n, w.data(), pr);
+        if (ok && (walk == SPM_INT_WALK_PRUNED || prune_preferred(a, n, pr))) {
+            rc = make_prune_plan(pr, n, lb, halved, device, out);
+            // no room for its lists: the other walks need next to nothing
+            if (rc != SPM_ENOMEM || walk == SPM_INT_WALK_PRUNED) return rc;
+        }
+        if (walk == SPM_INT_WALK_PRUNED) return SPM_ERANGE;
+    }
     const bool sp = walk == SPM_INT_WALK_SPARSE || (walk == SPM_INT_WALK_AUTO && int_sparse_preferred(a, n));
     const bool fp = !sp && (walk == SPM_INT_WALK_FP64 || (walk == SPM_INT_WALK_AUTO && small));
     std::vector<int64_t> sorted;
@@ -699,6 +792,28 @@ static int dense_run(spm_plan* p, hipStream_t st, spm_result* r)
     return SPM_OK;
 }
 
+// The launches of a pruned plan over the first launch's prefixes [tb, te):
+// one per column group from first_group - 1 down to 2, then the nodes.
+static int prune_launch(spm_plan* p, uint64_t tb, uint64_t te, hipStream_t st)
+{
+    unsigned long long* list = nullptr;
+    unsigned int* count = nullptr;
+    unsigned long long* partial = (unsigned long long*)p->d_partial;
+    for (int group = p->first_group - 1; group >= 1; --group) {
+        unsigned long long* out = p->d_list[group & 1];
+        unsigned int* out_count = p->d_counter + (size_t)kPruneSets * kPruneCounterStride * (group - 1);
+        void* args[] = {&p->d_M, &list, &count, &out, &out_count, &p->list_cap, &group, &partial, &tb, &te};
+        const int grid = group == 1 ? p->grid2 : p->grid;
+        if (hipLaunchKernel(group == 1 ? p->kern2 : p->kern, dim3(grid), dim3(p->block), args, p->lds_bytes, st) !=
+            hipSuccess)
+            return SPM_EHIP;
+        list = out;
+        count = out_count;
+        partial += 2 * (size_t)grid;
+    }
+    return SPM_OK;
+}
+
 static int int_run(spm_plan* p, hipStream_t st, spm_result* r)
 {
     const double t0 = now_seconds();
@@ -711,7 +826,10 @@ static int int_run(spm_plan* p, hipStream_t st, spm_result* r)
         uint64_t tb = per * s, te = std::min<uint64_t>(p->tasks, per * (s + 1));
         if (tb >= te) break;
         int acc = s > 0 ? 1 : 0;
-        if (p->kind == 4) {
+        if (p->d_counter) {
+            const int rc = prune_launch(p, tb, te, st);
+            if (rc != SPM_OK) return rc;
+        } else if (p->kind == 4) {
             void* args[] = {&p->d_partial, &tb, &te, &p->chunks, &p->L, &acc};
             if (hipModuleLaunchKernel(p->fn, p->grid, 1, 1, kDenseBlock, 1, 1, 0, st, args, nullptr) != hipSuccess)
                 return SPM_EHIP;
@@ -723,10 +841,10 @@ static int int_run(spm_plan* p, hipStream_t st, spm_result* r)
         ++launches;
     }
     {
-        int nrec = p->grid;
-        void* args[] = {&p->d_partial, &nrec, &p->d_out};
-        if (hipLaunchKernel(reduce_i128_kernel_ptr(), dim3(1), dim3(256), args, 0, st) != hipSuccess)
-            return SPM_EHIP;
+        int nrec = p->d_counter ? p->partial_cap : p->grid, counters = kPruneSets * p->first_group;
+        void* args[] = {&p->d_partial, &nrec, &p->d_out, &p->d_counter, &counters};
+        const void* k = p->d_counter ? reduce_prune_kernel_ptr() : reduce_i128_kernel_ptr();
+        if (hipLaunchKernel(k, dim3(1), dim3(256), args, 0, st) != hipSuccess) return SPM_EHIP;
     }
     if (hipEventRecord(p->ev1, st) != hipSuccess) return SPM_EHIP;
     if (hipMemcpyAsync(p->h_out, p->d_out, 16, hipMemcpyDeviceToHost, st) != hipSuccess) return SPM_EHIP;
@@ -765,7 +883,7 @@ extern "C" int spm_plan_info(const spm_plan* p, int* grid, int* block, int* log2
 {
     if (!p) return SPM_EINVAL;
     if (grid) *grid = p->grid;
-    if (block) *block = kDenseBlock;
+    if (block) *block = p->block;
     if (log2_chunk) *log2_chunk = p->L;
     if (tasks) *tasks = p->tasks;
     return SPM_OK;

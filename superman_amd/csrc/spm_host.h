@@ -15,7 +15,7 @@ namespace spm {
 constexpr int kWaveLanes = 64;
 
 int device_cus(int device, int* cus);
-int blocks_per_cu(int device, const void* kern, int block, int* bpc);
+int blocks_per_cu(int device, const void* kern, int block, int* bpc, int lds_bytes = 0);
 double now_seconds();
 
 // Gray-walk geometry shared by the dense kernels: 2^L steps per lane chunk,
@@ -87,6 +87,21 @@ int f32prod_scale_exponent(int n);
 int f32prod_scale(const double* a, int n, double* scaled);
 void f32prod_finish(int n, int log2_scale, spm_result* r);
 int int_fill_result(int n, unsigned long long lo, unsigned long long hi, spm_result* r, int halved_rows = 0);
+
+// prune.cpp -- layout of an integer matrix for int_prune_kernel: false when
+// its row sums do not fit packed fields (or the order is below kPruneMinN).
+constexpr int kPruneMinN = 13;
+constexpr int kPruneAutoN = 24;  // below, the walks take under 0.04 ms and a launch more decides
+struct PrunePlan {
+    int field_bytes = 1, dwords = 4, lds_bytes = 0;
+    int first_group = 2;     // the first launch's prefixes set the groups from this one outward
+    uint64_t prefixes = 0;   // and are this many
+    double nodes = 0;  // estimated nodes of 4096 subsets visited
+    double upper = 0;  // and of the groups above them
+    std::vector<int> blob;
+};
+bool prune_plan(const int64_t* a, int n, const unsigned char* w, PrunePlan& p);
+bool prune_preferred(const int64_t* a, int n, const PrunePlan& p);
 
 // codegen.cpp -- SpaRyser per-pattern kernels
 void ut_order_mask(const unsigned char* nz, int n, std::vector<int>& rowPerm, std::vector<int>& colPerm);

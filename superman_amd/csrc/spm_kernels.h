@@ -4,6 +4,7 @@
 // host stub address, launched with hipLaunchKernel by the drivers.
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 namespace spm {
@@ -60,6 +61,56 @@ int int_small_bits(int n);
 const void* int_sparse_kernel_ptr(int n);
 constexpr int kSparseRec = 16;   // ints per record
 constexpr int kSparseSlots = 7;  // entries per record
+
+// int_prune.hip -- exact sum over the subsets with no zero row
+// (walk_prune.h).
+//   args: (const int* blob, const unsigned long long* in, const unsigned int*
+//          in_count, unsigned long long* out, unsigned int* out_count,
+//          unsigned int cap, int group, unsigned long long* partial
+//          /* [grid][2], its own for each launch */, uint64_t begin, uint64_t
+//          end), kPruneBlock threads, dynamic LDS PrunePlan::lds_bytes, a
+//          grid of at least kPruneSets waves in every launch but those of a
+//          run of one launch.  Launch k of a run takes prefixes
+//          of the groups above `group` (in_count null: all settings, [begin,
+//          end), end - begin a power of two) and lists the survivors of
+//          group's settings in `out`; the last one (nodes true, group 1)
+//          walks the listed nodes, with out_count as its work counters.
+//          Lists have kPruneSets segments of cap prefixes; a set of counters
+//          is kPruneSets lines, all 0 before the run.
+//   reduce: (const unsigned long long* partial, int nrec, unsigned long long*
+//          out /* [2] */, unsigned int* counter, int counters), which sets
+//          the counters back to 0
+// field_bytes 1 (dwords 4, 8, 12, 16) or 2 (dwords 8, 16, 24).
+const void* int_prune_kernel_ptr(int field_bytes, int dwords, bool nodes);
+const void* reduce_prune_kernel_ptr();
+constexpr int kPruneBlock = 512;
+constexpr int kPruneLevels = 12;      // column groups of 6 of 62 walked columns, and one
+constexpr int kPruneTopBits = 15;     // the first launch has at most 2^15 prefixes
+constexpr int kPruneSets = 64;        // counters per launch, one 64-byte line each
+constexpr int kPruneCounterStride = 16;
+constexpr int kPruneEntriesMax = 2048;  // zero masks (8 bytes each)
+constexpr size_t kPruneStaticLds = (kPruneBlock / 64) * (16 + 8 * kPruneLevels + 2048);
+constexpr size_t kPruneLdsMax = 65536;
+// The blob (ints): the header slots, then sections at places that depend on
+// the template's dwords and fields only, so that the kernel's scalar loads
+// of them need no offset loaded first.
+enum PruneSlot {
+    kPruneGroups,   // column groups of 6
+    kPruneLeaf,     // leading fields that have zero masks (a multiple of two dwords' fields)
+    kPruneTested,   // those of them that are tested (the masks of the others are 0)
+    kPruneStride,   // zero masks per field
+    kPruneMode,     // product()
+    kPruneBits,     // walked columns, n - 1
+    kPruneUsed = 8,                               // [kPruneLevels] dwords with a nonzero care mask
+    kPruneZero = kPruneUsed + kPruneLevels        // [dwords] packed zero pattern, -o; then:
+};
+constexpr int prune_offset_at(int dwords) { return kPruneZero + dwords; }              // [fields] o: y = field + o
+constexpr int prune_care_at(int dwords, int fields) { return prune_offset_at(dwords) + fields; }  // [kPruneLevels][dwords]
+constexpr int prune_on_at(int dwords, int fields)     // [kMaxN][2][dwords] a column's fields: in the subset, out of it
+{
+    return prune_care_at(dwords, fields) + kPruneLevels * dwords;
+}
+constexpr int prune_blob_ints(int dwords, int fields) { return prune_on_at(dwords, fields) + kMaxN * 2 * dwords; }
 
 // Generated SpaRyser kernels walk 2^3-step blocks with L > 3.
 constexpr int kCodegenMinN = 5;
