@@ -44,6 +44,7 @@ SOURCES = [  # the longest compiles first, so that the job pool starts them earl
     ("int_sparse_17.hip", []),
     ("batch.hip", []),
     ("int_dense.hip", []),
+    ("dense_pair.hip", []),
     ("dense_f64.hip", []),
     ("int_sparse.hip", []),
     ("int_small.hip", []),

@@ -144,6 +144,14 @@ void gray_geometry(int n, int unroll_bits, int64_t resident_waves, int* L, uint6
     *tasks = (*chunks + kWaveLanes - 1) / kWaveLanes;
 }
 
+void pair_geometry(int n, int64_t resident_waves, int* L, uint64_t* chunks, uint64_t* tasks)
+{
+    gray_geometry(n, dense_f64_unroll_bits(n), resident_waves, L, chunks, tasks, GrayWalk::kReal);
+    *L = std::max(*L, kPairMinChunk);
+    *chunks = uint64_t(1) << (n - 1 - *L);
+    *tasks = (*chunks + kWaveLanes - 1) / kWaveLanes;
+}
+
 }  // namespace spm
 
 using namespace spm;
@@ -170,6 +178,8 @@ struct spm_plan {
     double* d_x0 = nullptr;
     double log2_bound = 0;   // integer kind: log2 of the bound on |T|
     int halved = 0;          // integer kinds: rows carried halved (int_row_weights)
+    bool pair = false;       // dense real plans: the matrix is scaled for dense_pair_kernel
+    PairScale scale;
     int log2_scale = 0;      // FP32-product plans: perm = 2^log2_scale perm(scaled)
     double* d_partial = nullptr;
     double* d_out = nullptr;
@@ -235,6 +245,21 @@ static void dense_grid(spm_plan* p)
     dense_launch_shape(p->kind, p->n, p->precision, p->tasks, p->max_grid, &p->grid, &p->slices);
 }
 
+static void dense_kernel_name(spm_plan* p)
+{
+    const char* comp = p->precision == SPM_PREC_COMPENSATED ? "true" : "false";
+    const int n = p->n, ub = dense_f64_unroll_bits(n);
+    char kn[96];
+    if (p->precision == SPM_PREC_F32_PRODUCT) std::snprintf(kn, sizeof kn, "dense_f32p_kernel<%d, %d>", n, ub);
+    else if (p->kind == 2) std::snprintf(kn, sizeof kn, "dense_c128_kernel<%d, %s>", n, comp);
+    else
+        std::snprintf(kn, sizeof kn, "%s<%d, %d, %s>",
+                      p->kern == dense_pair_kernel_ptr(n, p->precision == SPM_PREC_COMPENSATED) ? "dense_pair_kernel"
+                                                                                                : "dense_f64_kernel",
+                      n, ub, comp);
+    p->kname = kn;
+}
+
 // Dense plans, real (kind 1) and complex (kind 2).  `a` is row-major n x n,
 // doubles or interleaved (re, im) pairs.
 static int make_dense_plan(int kind, const double* a, int n, int precision, int device, spm_plan** out)
@@ -261,7 +286,10 @@ static int make_dense_plan(int kind, const double* a, int n, int precision, int 
     p->precision = precision;
     p->device = device;
     const bool comp = precision == SPM_PREC_COMPENSATED;
-    p->kern = f32p ? dense_f32p_kernel_ptr(n) : kind == 1 ? dense_f64_kernel_ptr(n, comp) : dense_c128_kernel_ptr(n, comp);
+    std::vector<double> scaled((size_t)(kind == 1 ? n * n : 0));
+    p->pair = kind == 1 && !f32p && pair_prepare(a, n, scaled.data(), &p->scale);
+    if (p->pair) a = scaled.data();
+    p->kern = p->pair ? dense_pair_kernel_ptr(n, comp) : f32p ? dense_f32p_kernel_ptr(n) : kind == 1 ? dense_f64_kernel_ptr(n, comp) : dense_c128_kernel_ptr(n, comp);
     p->rec = kind == 1 ? 4 : 8;
     p->comps = kind == 1 ? 1 : 2;
     if (!p->kern) {
@@ -276,24 +304,17 @@ static int make_dense_plan(int kind, const double* a, int n, int precision, int 
     }
     const int64_t waves = int64_t(bpc) * cus * (kDenseBlock / kWaveLanes);
     const int ub = kind == 1 ? dense_f64_unroll_bits(n) : (n >= 3 ? 1 : 0);
-    gray_geometry(n, ub, waves, &p->L, &p->chunks, &p->tasks, kind == 1 ? GrayWalk::kReal : GrayWalk::kComplex);
+    if (p->pair) pair_geometry(n, waves, &p->L, &p->chunks, &p->tasks);
+    else gray_geometry(n, ub, waves, &p->L, &p->chunks, &p->tasks, kind == 1 ? GrayWalk::kReal : GrayWalk::kComplex);
     p->max_grid = bpc * cus;
     dense_grid(p);
-    char kn[96];
-    if (f32p)
-        std::snprintf(kn, sizeof kn, "dense_f32p_kernel<%d, %d>", n, ub);
-    else if (kind == 1)
-        std::snprintf(kn, sizeof kn, "dense_f64_kernel<%d, %d, %s>", n, ub, comp ? "true" : "false");
-    else
-        std::snprintf(kn, sizeof kn, "dense_c128_kernel<%d, %s>", n, comp ? "true" : "false");
-    p->kname = kn;
+    dense_kernel_name(p);
 
     // Host preparation (dpSingleGPU.cuh:62-82; gpuComputeComplex.cu:212-241).
     const size_t col = (size_t)w * n;   // doubles per column
     const size_t plane = col * n;
-    std::vector<double> colmaj(2 * plane), x0(col), scaled;
+    std::vector<double> colmaj(2 * plane), x0(col);
     if (f32p) {
-        scaled.resize((size_t)n * n);
         p->log2_scale = f32prod_scale(a, n, scaled.data());
         a = scaled.data();
     }
@@ -781,6 +802,7 @@ static int dense_run(spm_plan* p, hipStream_t st, spm_result* r)
 
     std::memset(r, 0, sizeof *r);
     const int n = p->n;
+    if (p->pair) pair_finish(p->scale, p->h_out);
     dense_fill_result(n, p->comps == 2, p->precision != SPM_PREC_PLAIN, p->h_out, r);
     if (p->precision == SPM_PREC_F32_PRODUCT) f32prod_finish(n, p->log2_scale, r);
     r->status = SPM_OK;
@@ -898,6 +920,11 @@ extern "C" int spm_plan_set_log2_chunk(spm_plan* p, int L)
     const int ub = p->kind == 1 ? dense_f64_unroll_bits(n) : (n >= 3 ? 1 : 0);
     const int lo = ub > 0 ? ub + 1 : (B >= 1 ? 1 : 0);
     if (L < lo || L > B) return SPM_EINVAL;
+    if (p->pair) {  // the scaled matrix by either kernel: shorter chunks one subset at a time
+        const bool comp = p->precision == SPM_PREC_COMPENSATED;
+        p->kern = L >= kPairMinChunk ? dense_pair_kernel_ptr(n, comp) : dense_f64_kernel_ptr(n, comp);
+        dense_kernel_name(p);
+    }
     p->L = L;
     p->chunks = uint64_t(1) << (B - L);
     p->tasks = (p->chunks + kWaveLanes - 1) / kWaveLanes;

@@ -3,54 +3,13 @@
 // Replaces the reference's dense GPU kernels
 // (Algorithms/GPU/Dense/DenseKernelDefinitions.cuh:37-552: xRegisterMShared,
 // xRegisterMSharedKahan and their placement variants).  The per-chunk walk is
-// in walk_f64.h; this file holds the grid-strided task loop over one
-// matrix's chunks, the block reduction into per-block records and the final
+// in walk_f64.h, the grid-strided task loop and the block reduction in
+// dense_chunks.h; this file holds the kernels that take a matrix as it is
+// (those with a column to scale to ones are dense_pair.hip's) and the final
 // reduction kernel.
-#include "walk_f64.h"
+#include "dense_chunks.h"
 
 namespace spm {
-
-// The grid-strided task loop over one matrix's chunks and the block
-// reduction into per-block records, for the accumulation policy Term.
-template <int N, int U, class Term>
-__device__ __forceinline__ void dense_chunks(const double* __restrict__ M, const double* __restrict__ x0,
-                                             double* __restrict__ partial, uint64_t task_begin,
-                                             uint64_t task_end, uint64_t num_chunks, int L, int accumulate)
-{
-    constexpr bool COMP = Term::kCompensated;
-    __shared__ double red[3 * (kDenseBlock / kWave)];
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint64_t wave = (uint64_t)blockIdx.x * (kDenseBlock / kWave) + (threadIdx.x / kWave);
-    const uint64_t nwave = (uint64_t)gridDim.x * (kDenseBlock / kWave);
-
-    double acc_hi = 0.0, acc_lo = 0.0, acc_abs = 0.0;
-    for (uint64_t task = task_begin + wave; task < task_end; task += nwave) {
-        const uint64_t h = task * kWave + lane;
-        const bool active = h < num_chunks;  // lanes past the end walk a dummy chunk
-        Term term;
-        real::walk_gray<N, U>(M, x0, h, L, term);
-        if (active) {
-            if constexpr (COMP) {
-                dd_add(acc_hi, acc_lo, term.t_hi, term.t_lo);
-                acc_abs += term.t_abs;
-            } else {
-                acc_hi += term.t_hi;
-            }
-        }
-    }
-    block_reduce_dd(acc_hi, acc_lo, acc_abs, red);
-    if (threadIdx.x == 0) {
-        double* out = partial + 4 * blockIdx.x;
-        if (accumulate) {  // later slice of a long run: add onto this block's record
-            dd_add(acc_hi, acc_lo, out[0], out[1]);
-            acc_abs += out[2];
-        }
-        out[0] = acc_hi;
-        out[1] = acc_lo;
-        out[2] = acc_abs;
-        out[3] = 0.0;
-    }
-}
 
 template <int N, int U, bool COMP>
 __global__ void __launch_bounds__(kDenseBlock) __attribute__((amdgpu_waves_per_eu(real::kDenseWaves<N>)))

@@ -52,7 +52,8 @@ constexpr int kMaxDevices = 64;
 struct DeviceState {
     double* base = nullptr;       // device address of `scratch` on this device
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    int bpc[kMaxN + 1][3] = {};   // resident blocks per CU by order and kernel (plain, compensated, FP32-product)
+    int bpc[kMaxN + 1][5] = {};   // resident blocks per CU by order and kernel (plain, compensated, FP32-product,
+                                  // then the pair kernel's plain and compensated)
 };
 
 std::mutex g_mu;
@@ -114,14 +115,20 @@ extern "C" int spm_dense_f64_noalloc(const double* a, int n, int precision, int 
     if ((st = device_setup(device, &d)) != SPM_OK) return out->status = st;
 
     // The geometry of spm_dense_f64 (make_dense_plan + dense_grid in capi.cpp).
-    const void* kern = f32p ? dense_f32p_kernel_ptr(n) : dense_f64_kernel_ptr(n, comp);
+    double scaled[kMaxN * kMaxN];
+    PairScale scale;
+    const bool pair = !f32p && pair_prepare(a, n, scaled, &scale);
+    if (pair) a = scaled;
+    const void* kern = pair ? dense_pair_kernel_ptr(n, comp)
+                            : f32p ? dense_f32p_kernel_ptr(n) : dense_f64_kernel_ptr(n, comp);
     if (!kern) return out->status = SPM_EINVAL;
     int bpc = 0;
-    if ((st = resident_blocks(*d, n, f32p ? 2 : comp ? 1 : 0, kern, &bpc)) != SPM_OK) return out->status = st;
+    if ((st = resident_blocks(*d, n, (pair ? 3 : 0) + (f32p ? 2 : comp ? 1 : 0), kern, &bpc)) != SPM_OK) return out->status = st;
     const int64_t waves = int64_t(bpc) * cus * (kDenseBlock / kWaveLanes);
     int L = 0;
     uint64_t chunks = 0, tasks = 0;
-    gray_geometry(n, dense_f64_unroll_bits(n), waves, &L, &chunks, &tasks, GrayWalk::kReal);
+    if (pair) pair_geometry(n, waves, &L, &chunks, &tasks);
+    else gray_geometry(n, dense_f64_unroll_bits(n), waves, &L, &chunks, &tasks, GrayWalk::kReal);
     int grid = 0, slices = 1;
     dense_launch_shape(1, n, precision, tasks, bpc * cus, &grid, &slices);
     if (grid > kMaxBlocks) return out->status = SPM_ENOMEM;  // more per-block records than the array holds
@@ -129,7 +136,6 @@ extern "C" int spm_dense_f64_noalloc(const double* a, int n, int precision, int 
     // Host preparation on the stack (dpSingleGPU.cuh:62-82), as spm_dense_f64.
     double planes[2 * kMaxN * kMaxN];
     double x0[kMaxN];
-    double scaled[kMaxN * kMaxN];
     int log2_scale = 0;
     if (f32p) {
         log2_scale = f32prod_scale(a, n, scaled);
@@ -171,6 +177,7 @@ extern "C" int spm_dense_f64_noalloc(const double* a, int n, int precision, int 
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, d->ev0, d->ev1) != hipSuccess) ms = -1.f;
 
+    if (pair) pair_finish(scale, rec);
     dense_fill_result(n, false, precision != SPM_PREC_PLAIN, rec, out);
     if (f32p) f32prod_finish(n, log2_scale, out);
     out->status = SPM_OK;

@@ -35,6 +35,110 @@ void dense_prepare(const double* a, int n, int w, double* planes, double* x0)
     }
 }
 
+namespace {
+
+// Whether sums of a row's entries are exact in FP64 (entries of few bits, such
+// as integers): then x has no rounding to lose.
+bool exact_sums(const double* a, int n)
+{
+    int top = -5000, low = 5000;
+    for (int e = 0; e < n * n; ++e) {
+        if (a[e] == 0.0) continue;
+        int x;
+        const int64_t m = (int64_t)std::ldexp(std::frexp(a[e], &x), 53);
+        top = std::max(top, x);
+        low = std::min(low, x - 53 + __builtin_ctzll((unsigned long long)m));
+    }
+    return top + 7 - low <= 53;  // 2 n entries and a half
+}
+
+bool power_of_two(double v)
+{
+    int x;
+    return std::fabs(std::frexp(v, &x)) == 0.5;
+}
+
+}  // namespace
+
+// The matrix with the rows divided by the entries c_i of one column, which
+// comes first and is all ones (PairTerm, walk_f64.h): perm(a) = prod c_i
+// perm(out).  A row's quotients are rounded once, a relative 2^-53 of each
+// entry.  The column is the one whose smallest |c_i| / max_j |a_ij| is the
+// largest, so the quotients stay near 1.  False, and the matrix is walked
+// as it is, when
+//   - every column has a zero (or an entry 2^-60 of its row's largest), or
+//     the row bounds sum_j |a_ij| / |c_i| multiply past 2^900 (products near
+//     overflow);
+//   - the row sums are exact as they are (integers, say) and the quotients
+//     would not be: a column of powers of two is taken there, or none.
+bool pair_prepare(const double* a, int n, double* out, PairScale* scale)
+{
+    if (n < kPairMinN) return false;
+    const bool exact = exact_sums(a, n);
+    double rowmax[kMaxN];
+    for (int i = 0; i < n; ++i) {
+        rowmax[i] = 0.0;
+        for (int j = 0; j < n; ++j) rowmax[i] = std::max(rowmax[i], std::fabs(a[(size_t)i * n + j]));
+        if (rowmax[i] == 0.0) return false;
+    }
+    int col = -1;
+    double best = 0x1p-60;
+    for (int j = 0; j < n; ++j) {
+        double least = 1.0;
+        bool two = true;
+        for (int i = 0; i < n && least > best; ++i) {
+            const double v = a[(size_t)i * n + j];
+            least = std::min(least, std::fabs(v) / rowmax[i]);
+            two = two && (!exact || power_of_two(v));
+        }
+        if (least > best && two) {
+            best = least;
+            col = j;
+        }
+    }
+    if (col < 0) return false;
+    double bound = 0.0, sh = 1.0, sl = 0.0;
+    int exp2 = 0;
+    for (int i = 0; i < n; ++i) {
+        const double* r = a + (size_t)i * n;
+        const double c = r[col];
+        double sum = 0.0;
+        for (int j = 0; j < n; ++j) {
+            const double v = r[j == 0 ? col : j == col ? 0 : j];
+            sum += std::fabs(v / c);
+            out[(size_t)i * n + j] = v / c;
+        }
+        bound += std::log2(sum);
+        int x;
+        const double m = std::frexp(c, &x);
+        exp2 += x;
+        const double p = sh * m;  // (sh, sl) *= m in double-double
+        const double e = std::fma(sh, m, -p) + sl * m;
+        sh = p + e;
+        sl = e - (sh - p);
+        const double f = std::frexp(sh, &x);
+        sl = std::ldexp(sl, -x);
+        sh = f;
+        exp2 += x;
+    }
+    if (!(bound <= 900.0)) return false;
+    scale->hi = sh;
+    scale->lo = sl;
+    scale->exp2 = exp2;
+    return true;
+}
+
+// rec = (hi, lo, abs) times the scale.
+void pair_finish(const PairScale& s, double* rec)
+{
+    const double p = rec[0] * s.hi;
+    const double e = std::fma(rec[0], s.hi, -p) + (rec[0] * s.lo + rec[1] * s.hi);
+    const double h = p + e;
+    rec[1] = std::ldexp(std::isfinite(h) ? e - (h - p) : 0.0, s.exp2);
+    rec[0] = std::ldexp(h, s.exp2);
+    rec[2] = std::ldexp(rec[2] * std::fabs(s.hi), s.exp2);
+}
+
 // Integer entry checks: |a| <= 2^30 and absolute row sums < 2^30 (so |y|
 // fits int32), y0 = y(empty set), and log2 of the bound on
 // |T| = 2^(n-1-e) |perm| (e = rows carried halved, int_row_weights):

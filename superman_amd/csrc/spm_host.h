@@ -25,6 +25,8 @@ double now_seconds();
 enum class GrayWalk { kOther, kReal, kComplex };
 void gray_geometry(int n, int unroll_bits, int64_t resident_waves, int* L, uint64_t* chunks, uint64_t* tasks,
                    GrayWalk walk = GrayWalk::kOther);
+// The same for dense_pair_kernel, whose chunks are at least 2^kPairMinChunk.
+void pair_geometry(int n, int64_t resident_waves, int* L, uint64_t* chunks, uint64_t* tasks);
 // Grid and launch slices of a dense walk over `tasks` wave tasks (kind 1
 // real, 2 complex, 5 generated real): as many blocks as the tasks fill, at
 // most max_grid (the resident ones); runs longer than ~4 s of VALU work are
@@ -62,6 +64,14 @@ inline double f32prod_err_est(int n, double abs_sum)
 
 // prep.cpp -- per-matrix host preparation and result conversion
 void dense_prepare(const double* a, int n, int w, double* planes, double* x0);
+// Matrices for dense_pair_kernel: column 0 of the scaled matrix is all ones,
+// perm(a) = (hi + lo) 2^exp2 perm(scaled).
+struct PairScale {
+    double hi = 1.0, lo = 0.0;
+    int exp2 = 0;
+};
+bool pair_prepare(const double* a, int n, double* scaled, PairScale* scale);
+void pair_finish(const PairScale& scale, double* rec);
 // w: per-row weights from int_row_weights (1 = row carried halved, 2 =
 // not); nullptr = every row 2 (the batch engine's layout).
 int int_row_weights(const int64_t* a, int n, unsigned char* w);

@@ -246,6 +246,55 @@ struct FpTerm {
     }
 };
 
+// Two subsets per step, for a matrix whose column 0 is all ones (pair_prepare
+// scales rows so): the walk visits the subsets without column 0, and each x
+// gives its own term and that of x + 1,
+//   prod_i x_i  and  prod_i (x_i + 1),  p <- p x_i  and  q <- fma(q, x_i, q),
+// so column 0 is never added to x: per two subsets n adds, n multiplies and
+// n FMAs instead of 2n adds and 2n multiplies, and q (x_i + 1) is rounded
+// once instead of twice.  add(x, negative) takes (-1)^m (P - Q).
+template <int N, bool COMP>
+struct PairTerm {
+    static constexpr bool kCompensated = COMP;
+    double t_hi = 0.0, t_lo = 0.0, t_abs = 0.0;
+    double blk = 0.0, blk_abs = 0.0;
+    __device__ __forceinline__ void add(const double (&x)[N], bool negative)
+    {
+        constexpr int H = N - 1;
+        static_assert(H >= 4, "four chains");
+        double p[4], q[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            p[k] = x[k];
+            q[k] = x[k] + 1.0;
+        }
+#pragma unroll
+        for (int r = 4; r < H; ++r) {
+            p[r & 3] *= x[r];
+            q[r & 3] = __builtin_fma(q[r & 3], x[r], q[r & 3]);
+        }
+        const double P = (p[0] * p[1]) * (p[2] * p[3]), Q = (q[0] * q[1]) * (q[2] * q[3]);
+        const double t = __builtin_fma(Q, x[H], Q);
+        blk = __builtin_fma(negative ? -P : P, x[H], blk);
+        blk = negative ? blk + t : blk - t;
+        if constexpr (COMP) {
+            blk_abs = __builtin_fma(__builtin_fabs(P), __builtin_fabs(x[H]), blk_abs);
+            blk_abs += __builtin_fabs(t);
+        }
+    }
+    __device__ __forceinline__ void fold()
+    {
+        if constexpr (COMP) {
+            dd_add_d(t_hi, t_lo, blk);
+            t_abs += blk_abs;
+        } else {
+            t_hi += blk;
+        }
+        blk = 0.0;
+        blk_abs = 0.0;
+    }
+};
+
 // FP32 products for nonnegative matrices whose rows the host scaled by
 // powers of two so that every |x_i| < 2^(c+1) with (c+1) N <= 127: x stays
 // FP64 (exact updates), the first N-1 factors are rounded to FP32 and
@@ -277,9 +326,10 @@ struct F32ProdTerm {
     }
 };
 
-// One lane's chunk: the 2^L Gray steps starting at k = h 2^L, every term
-// handed to `term`.
-template <int N, int U, class Term>
+// One lane's chunk: the 2^L Gray steps starting at k = h 2^L over the walked
+// columns 0..NC-1 of M (column stride N), every term handed to `term`, which
+// folds FOLD steps at a time.
+template <int N, int U, class Term, int NC = N - 1, uint32_t FOLD = kFoldSteps>
 __device__ __forceinline__ void walk_gray(const double* __restrict__ M,   // [2][N][N]: +A, -A
                                           const double* __restrict__ x0,  // x(empty set)
                                           uint64_t h, int L, Term& term)
@@ -295,7 +345,7 @@ __device__ __forceinline__ void walk_gray(const double* __restrict__ M,   // [2]
     }
     const uint64_t k0 = h << L;
     const uint64_t g0 = k0 ^ (k0 >> 1);
-    for (int j = (L > 0 ? L - 1 : 0); j < N - 1; ++j) {
+    for (int j = (L > 0 ? L - 1 : 0); j < NC; ++j) {
         const double b = ((g0 >> j) & 1u) ? 1.0 : 0.0;
         const const_f64* __restrict__ col = step_column(M + j * N);
 #pragma unroll
@@ -320,7 +370,7 @@ __device__ __forceinline__ void walk_gray(const double* __restrict__ M,   // [2]
             return (((m >> (tz + 1)) & 1u) ? Mneg : M) + (tz + 1) * N;
         };
         const uint32_t half = nblk >> 1;
-        constexpr uint32_t G = kFoldSteps / 2;
+        constexpr uint32_t G = FOLD / 2;
         Column<N> ca, cb;
         term.add(x, false);  // k = 0: the chunk start
         load_column(cb, M);                          // k = 1: +column 0
@@ -339,7 +389,7 @@ __device__ __forceinline__ void walk_gray(const double* __restrict__ M,   // [2]
             term.add(x, false);
             step_fence();
             add_column(x, cb);
-            load_column(ca, a_col(m + 1));  // m+1 = nblk loads column L <= N-1: harmless
+            load_column(ca, a_col(m + 1));  // m+1 = nblk loads column L <= NC: harmless
             step_fence();
             term.add(x, true);
             step_fence();
@@ -360,7 +410,7 @@ __device__ __forceinline__ void walk_gray(const double* __restrict__ M,   // [2]
         // Unpipelined walk (U = 0: tiny orders; U >= 2: tuning builds).
         // Block m starts with the flip of the runtime column ctz(m) + U;
         // its other steps flip compile-time columns.
-        constexpr uint32_t G = (kFoldSteps >> U) > 0 ? (kFoldSteps >> U) : 1;
+        constexpr uint32_t G = (FOLD >> U) > 0 ? (FOLD >> U) : 1;
         auto block_tail = [&](uint32_t m) __attribute__((always_inline)) {
             if constexpr (U > 0) {
                 // bit U of the step index.  Held in a VGPR: a VOP3 op takes
