@@ -637,10 +637,20 @@ extern "C" int spm_plan_codegen(const int64_t* a, int n, int options, int device
     }
     const int64_t waves = int64_t(bpc) * cus * (kDenseBlock / kWaveLanes);
     gray_geometry(n, codegen_int_unroll_bits(b.data(), n), waves, &p->L, &p->chunks, &p->tasks);
+    const bool pruned = gen_pruned(b.data(), n);
+    if (pruned) {
+        p->L = kGenPruneChunk;
+        p->chunks = uint64_t(1) << (n - 1 - p->L);
+        p->tasks = p->chunks / kWaveLanes;
+    }
     const uint64_t need_blocks = (p->tasks + (kDenseBlock / kWaveLanes) - 1) / (kDenseBlock / kWaveLanes);
     p->grid = (int)std::min<uint64_t>(uint64_t(bpc) * cus, need_blocks);
     const double est_s = std::ldexp(1.0, n - 1) * 16.0 / 3.9e13;
     p->slices = (int)std::min<double>(std::max(1.0, std::ceil(est_s / 4.0)), (double)p->tasks);
+    if (pruned) {  // a hundredth of the time; slices are a power of two of whole sieve prefixes
+        p->slices = 1;
+        while (p->slices < est_s / 400.0 && p->slices < 1 << 12) p->slices *= 2;
+    }
     SPM_TRY(hipMalloc(&p->d_partial, sizeof(unsigned long long) * 2 * p->grid));
     SPM_TRY(hipMalloc(&p->d_out, sizeof(double) * 6));
     SPM_TRY(hipHostMalloc(&p->h_out, sizeof(double) * 6, hipHostMallocDefault));

@@ -248,12 +248,61 @@ void emit_block_replay(std::ostringstream& o, int U, const char* M, const char* 
     o << ind << "}\n";
 }
 
+// A pruned kernel takes a chunk's prefix, the subset's columns >= L, through
+// three sieves before it walks the chunk: rows whose columns are all >= L + 12,
+// then >= L + 6, then >= L, each tested at the first level that fixes them and
+// each dropping every chunk below for good when zero (the term of every
+// subset there is).  The prefixes of a level are tested 64 at a time, one per
+// lane: 64 blocks (of 64 tasks), the 64 tasks of a live block, the 64 chunks of
+// a live task.  (Order 40 has 2^22 blocks: tested one by one in scalar code
+// they took 0.5 ms.)
+struct Sieve {
+    int level;              // columns below are not fixed yet
+    std::vector<int> rows;  // rows fixed at this level and not before
+};
+
+std::vector<Sieve> sieves(const std::vector<int64_t>& b, const std::vector<char>& zr, int n)
+{
+    std::vector<Sieve> v = {{kGenPruneChunk + 12, {}}, {kGenPruneChunk + 6, {}}, {kGenPruneChunk, {}}};
+    for (int r = 0; r < n; ++r) {
+        if (!zr[r]) continue;
+        int low = n;
+        for (int c = n - 2; c >= 0; --c)
+            if (b[(size_t)r * n + c] != 0) low = c;
+        for (Sieve& s : v)
+            if (low >= s.level) {
+                s.rows.push_back(r);
+                break;
+            }
+    }
+    return v;
+}
+
+// One sieve over the lanes' prefixes, which clears `alive`; g names the 64-bit
+// Gray prefix whose bits >= level are the subset's columns.  Leaves the
+// (outer) loop's round when no lane is left.
+void emit_sieve(std::ostringstream& o, const Sieve& s, const std::vector<int64_t>& wb, const std::vector<int64_t>& y0,
+                int n, const char* g, const char* ind)
+{
+    int k = 0;
+    for (int r : s.rows) {
+        o << ind << "{ int v = " << lit(y0[r]) << ";";
+        for (int c = s.level; c < n - 1; ++c) {
+            const int64_t d = wb[(size_t)r * n + c];
+            if (d != 0) o << " v += " << lit(d) << " & -(int)((" << g << " >> " << c << ") & 1ull);";
+        }
+        o << " alive = alive && v != 0; }\n";
+        if (++k % 4 == 0) o << ind << "if (__builtin_amdgcn_ballot_w64(alive) == 0) continue;\n";
+    }
+}
+
 }  // namespace
 
 std::string emit_int_kernel(const std::vector<int64_t>& b, int n, const std::string& name)
 {
     const bool compact = gen_compact_term(b.data(), n);
-    const int U = gen_unroll_bits_int(n, compact);
+    const bool prune = gen_pruned(b.data(), n);
+    const int U = codegen_int_unroll_bits(b.data(), n);
     // y = 2x, halved on rows with even sums (int_row_weights): wb holds the
     // walk's increments w_r b_rc
     std::vector<unsigned char> w(n);
@@ -279,14 +328,76 @@ std::string emit_int_kernel(const std::vector<int64_t>& b, int n, const std::str
     o << "\n";
     o << name << "(unsigned long long* __restrict__ partial, unsigned long long task_begin,\n"
       << "    unsigned long long task_end, unsigned long long num_chunks, int L, int accumulate)\n{\n";
-    o << "    __shared__ unsigned long long red[8];\n"
-         "    const unsigned lane = threadIdx.x & 63u;\n"
-         "    const unsigned long long wave = (unsigned long long)blockIdx.x * 4 + (threadIdx.x >> 6);\n"
-         "    const unsigned long long nwave = (unsigned long long)gridDim.x * 4;\n"
-         "    const bool idle = (unsigned long long)lane >= num_chunks;\n"
-         "    unsigned __int128 acc = 0;\n"
-         "    for (unsigned long long task = task_begin + wave; task < task_end; task += nwave) {\n"
-         "        const unsigned long long h = task * 64 + lane;\n";
+    if (!prune) {
+        o << "    __shared__ unsigned long long red[8];\n"
+             "    const unsigned lane = threadIdx.x & 63u;\n"
+             "    const unsigned long long wave = (unsigned long long)blockIdx.x * 4 + (threadIdx.x >> 6);\n"
+             "    const unsigned long long nwave = (unsigned long long)gridDim.x * 4;\n"
+             "    const bool idle = (unsigned long long)lane >= num_chunks;\n"
+             "    unsigned __int128 acc = 0;\n"
+             "    for (unsigned long long task = task_begin + wave; task < task_end; task += nwave) {\n"
+             "        const unsigned long long h = task * 64 + lane;\n";
+    } else {
+        // Blocks (in 2^cut parts when there are few) go to the waves in
+        // batches of up to 64, in the order of a bijection of their index
+        // (neighbouring prefixes survive alike).  bm and tm: the batch's
+        // parts and the part's tasks still to look into.  Live chunks wait
+        // in a queue per wave until 64 are walked together.
+        const std::vector<Sieve> sv = sieves(b, zr, n);
+        const int LC = kGenPruneChunk, bb = n - 1 - LC - 12, cut = std::min(6, std::max(0, 15 - bb));
+        const int pb = std::min(6, std::max(0, bb + cut - 13));  // log2 of a batch
+        o << "    __shared__ unsigned long long red[8];\n"
+             "    __shared__ unsigned long long live[4 * 128];\n"
+             "    const unsigned lane = threadIdx.x & 63u;\n"
+             "    const unsigned w0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);\n"
+             "    const unsigned long long nwave = (unsigned long long)gridDim.x * 4;\n"
+             "    const unsigned long long parts = (task_end - task_begin) >> " << 6 - cut << ";\n"
+             "    unsigned long long* const queue = live + w0 * 128;\n"
+             "    unsigned long long pi = (unsigned long long)blockIdx.x * 4 + w0, x = 0, T0 = 0, bm = 0, tm = 0;\n"
+             "    unsigned head = 0, tail = 0;\n"
+             "    unsigned __int128 total = 0;\n"
+             "    for (;;) {\n"
+             "        while (tail - head < 64u) {\n"
+             "            if (tm == 0) {\n"
+             "                if (bm == 0) {\n"
+             "                    if (pi >= parts >> " << pb << ") break;\n"
+             "                    bool alive = lane < " << (1 << pb) << "u;\n"
+             "                    x = (((pi << " << pb << ") + lane) * 0x9e3779b97f4a7c15ull) & (parts - 1);\n"
+             "                    x ^= x >> " << std::max(1, (bb + cut) / 2) << ";\n"
+             "                    x = task_begin + (((x * 0xbf58476d1ce4e5b9ull) & (parts - 1)) << " << 6 - cut << ");\n"
+             "                    pi += nwave;\n"
+             "                    const unsigned long long kb = x << " << LC + 6 << ", gb = kb ^ (kb >> 1);\n";
+        emit_sieve(o, sv[0], wb, y0, n, "gb", "                    ");
+        o << "                    bm = __builtin_amdgcn_ballot_w64(alive);\n"
+             "                    continue;\n"
+             "                }\n"
+             "                const int bl = __builtin_ctzll(bm);\n"
+             "                bm &= bm - 1;\n"
+             "                T0 = ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(x >> 32), bl) << 32) | "
+             "(unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, bl);\n"
+             "                bool alive = lane < " << (64 >> cut) << "u;\n"
+             "                const unsigned long long kt = (T0 + lane) << " << LC + 6 << ", gt = kt ^ (kt >> 1);\n";
+        emit_sieve(o, sv[1], wb, y0, n, "gt", "                ");
+        o << "                tm = __builtin_amdgcn_ballot_w64(alive);\n"
+             "                continue;\n"
+             "            }\n"
+             "            const unsigned long long hc = (T0 + __builtin_ctzll(tm)) * 64 + lane, kc = hc << " << LC
+          << ", gc = kc ^ (kc >> 1);\n"
+             "            tm &= tm - 1;\n"
+             "            bool alive = true;\n";
+        emit_sieve(o, sv[2], wb, y0, n, "gc", "            ");
+        o << "            const unsigned long long lm = __builtin_amdgcn_ballot_w64(alive);\n"
+             "            const unsigned at = __builtin_amdgcn_mbcnt_hi((unsigned)(lm >> 32), "
+             "__builtin_amdgcn_mbcnt_lo((unsigned)lm, tail));\n"
+             "            if (alive) queue[at & 127u] = hc;\n"
+             "            tail += (unsigned)__builtin_popcountll(lm);\n"
+             "        }\n"
+             "        if (tail == head) break;\n"
+             "        const unsigned count = min(64u, tail - head);\n"
+             "        const unsigned long long h = queue[(head + min(lane, count - 1u)) & 127u];\n"
+             "        head += count;\n"
+             "        unsigned __int128 acc = 0;\n";
+    }
     o << "        int ";
     for (int i = 0; i < n; ++i) o << "y" << i << " = " << lit(y0[i]) << (i + 1 < n ? ", " : ";\n");
     o << "        const unsigned long long k0 = h << L;\n"
@@ -355,7 +466,8 @@ std::string emit_int_kernel(const std::vector<int64_t>& b, int n, const std::str
     // bits of m from the lowest (half the blocks stop at the first test)
     o << "        for (unsigned m = 1; m < nblk; ++m) {\n"
          "            const int lmm = (m == half) ? lm : -(int)((m >> (__builtin_ctz(m) + 1)) & 1u);\n";
-    for (int c = U; c < n - 1 && c - U < 32; ++c) {
+    const int flips = prune ? std::min(n - 1, kGenPruneChunk) : n - 1;  // m has L - U bits
+    for (int c = U; c < flips && c - U < 32; ++c) {
         o << "            " << (c == U ? "if" : "} else if") << " (m & " << (1u << (c - U)) << "u) {\n";
         emit_flip_lane(o, wb, zr, n, c, "lmm", "                ");
     }
@@ -363,9 +475,14 @@ std::string emit_int_kernel(const std::vector<int64_t>& b, int n, const std::str
     emit_term(o, n, false, "            ", compact, true);
     block_tail("            ");
     o << "        }\n";
-    o << "    }\n"
-         "    if (idle) acc = 0;\n"
-         "    unsigned long long lo = (unsigned long long)acc, hi = (unsigned long long)(acc >> 64);\n"
+    if (prune)
+        o << "        if (lane < count) total += acc;\n"
+             "    }\n"
+             "    unsigned __int128 acc = total;\n";
+    else
+        o << "    }\n"
+             "    if (idle) acc = 0;\n";
+    o << "    unsigned long long lo = (unsigned long long)acc, hi = (unsigned long long)(acc >> 64);\n"
          "    for (int off = 32; off >= 1; off >>= 1) {\n"
          "        const unsigned long long olo = __shfl_xor(lo, off, 64);\n"
          "        const unsigned long long ohi = __shfl_xor(hi, off, 64);\n"
@@ -646,9 +763,44 @@ uint64_t real_pattern_hash(const double* b, int n, int options, int precision)
     return h;
 }
 
+// Whether an integer kernel is pruned: when the rows fixed outside a chunk
+// leave less than a quarter of the chunks live (by the row-independence
+// estimate; above that the sieves save less than walking 64 chunks that all
+// meet nonzero terms costs), and there are blocks of 64 tasks to share out.
+// Kernel ms at order 36 with 4, 6 and 8 entries per row and order 40 with 4
+// and 8 (0/1): unpruned 5.0 / 19 / 79 / 55 / 560, pruned 0.077 / 0.48 / 2.9 /
+// 0.106 / 12.1; order 24 with 4: 0.029 and 0.023.  The chunks are short (2^5
+// steps in blocks of 2^2): chunks of 2^9 took 3-5x as long, 2^7 1.3-1.9x, since
+// the less of a chunk is walked blind the fewer waves form a product for one
+// lane.
+bool gen_pruned(const int64_t* b, int n)
+{
+    if (n < 24) return false;  // 0.02 ms either way
+    double live = 1.0;
+    for (int r = 0; r < n; ++r) {
+        int64_t sum = 0;
+        int k = 0, low = n;
+        for (int c = n - 1; c >= 0; --c) {
+            sum += b[(size_t)r * n + c];
+            if (c < n - 1 && b[(size_t)r * n + c] != 0) {
+                ++k;
+                low = c;
+            }
+        }
+        if ((sum & 1) != 0 || low < kGenPruneChunk) continue;
+        double p = 1.0;  // C(k, floor(k/2)) / 2^k
+        for (int t = 1; t <= k; ++t) p *= (t <= k / 2 ? double(k - k / 2 + t) / t : 1.0) * 0.5;
+        live *= 1.0 - std::min(1.0, p);
+    }
+    return live < 0.25;
+}
 int codegen_real_unroll_bits(int n) { return gen_unroll_bits_real(n); }
 bool gen_compact_term(const int64_t* b, int n) { return int_nonzero_term_fraction(b, n) < kGenCompactTermQ; }
-int codegen_int_unroll_bits(const int64_t* b, int n) { return gen_unroll_bits_int(n, gen_compact_term(b, n)); }
+int codegen_int_unroll_bits(const int64_t* b, int n)
+{
+    if (gen_pruned(b, n)) return kGenPruneUnroll;
+    return gen_unroll_bits_int(n, gen_compact_term(b, n));
+}
 
 // FNV-1a over the pattern, values and generator options.
 uint64_t pattern_hash(const int64_t* b, int n, int options)

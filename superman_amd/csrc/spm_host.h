@@ -131,6 +131,11 @@ constexpr double kGenCompactTermQ = 5e-7;
 int gen_unroll_bits_int(int n, bool compact);
 bool gen_compact_term(const int64_t* b, int n);
 int codegen_int_unroll_bits(const int64_t* b, int n);
+// Integer kernels that test a chunk's prefix before they walk it, always with
+// chunks of 2^kGenPruneChunk steps and blocks of 2^kGenPruneUnroll.
+constexpr int kGenPruneChunk = 5;
+constexpr int kGenPruneUnroll = 2;
+bool gen_pruned(const int64_t* b, int n);
 int codegen_real_unroll_bits(int n);
 uint64_t pattern_hash(const int64_t* b, int n, int options);
 int codegen_get_kernel(int device, uint64_t hash, const std::string& src, const std::string& name, hipFunction_t* fn,
