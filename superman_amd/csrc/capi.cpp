@@ -746,6 +746,14 @@ extern "C" int spm_plan_codegen_real(const double* a, int n, int options, int pr
     }
     const int64_t waves = int64_t(bpc) * cus * (kDenseBlock / kWaveLanes);
     gray_geometry(n, codegen_real_unroll_bits(n), waves, &p->L, &p->chunks, &p->tasks);
+    if (const int m = real_elim_columns(b.data(), n)) {
+        // 4 to 64 outer steps per chunk, two chunks or more per lane
+        int lw = 0;
+        while ((int64_t(1) << lw) < waves) ++lw;
+        p->L = m + std::min(6, std::max(2, n - 1 - m - 6 - lw - 1));
+        p->chunks = uint64_t(1) << (n - 1 - p->L);
+        p->tasks = (p->chunks + kWaveLanes - 1) / kWaveLanes;
+    }
     p->max_grid = bpc * cus;
     dense_grid(p);
     SPM_TRY(hipMalloc(&p->d_partial, sizeof(double) * p->rec * p->grid));

@@ -43,6 +43,7 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <iterator>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -623,10 +624,350 @@ void emit_real_term(std::ostringstream& o, const RealLevels& lv, bool negative, 
       << ", S0, blk); ba = __builtin_fma(__builtin_fabs(P), __builtin_fabs(S0), ba); }\n";
 }
 
+// ---------------------------------------------------------------------------
+// Inner columns summed out.  With the columns >= m set, the sum over all
+// settings T of columns 0..m-1,
+//   E = sum_T (-1)^|T| prod_r x_r(T),
+// is a sum over m binary variables of a product of one factor per row, each
+// depending only on the few inner columns its row has entries in.  It is
+// formed one column at a time: the factors with column c are multiplied into
+// one table over their other columns and c's two settings subtracted.  The
+// cost grows with the tables (2^w entries, w columns tied together by shared
+// rows), not with 2^m: order 36 with 5 entries per row sums 2^11 subsets in
+// about 600 operations, 0.3 per subset against 9 for the walk.  The same
+// tables of absolute values, added instead of subtracted, give sum |term|;
+// a product of rows alone shares its value (|ab| = |a||b| as rounded).
+// ---------------------------------------------------------------------------
+struct Factor {
+    std::vector<int> scope;  // columns, ascending; entry i has column scope[k] set when bit k of i is
+    std::vector<std::string> val, abs;
+    bool pure = true;        // a product of rows: abs is |val|
+    int row = -1;            // a single row's, not written out yet (val and abs empty)
+};
+
+class Eliminator {
+public:
+    Eliminator(const std::vector<double>& b, int n, int m) : b_(b), n_(n), m_(m) {}
+
+    // Emits E into `P` and its absolute sum into `A`.  False when an inner
+    // column is empty.  ops: FP64 instructions; peak: table entries alive.
+    bool run(int& ops, int& peak, std::string* code, const char* ind)
+    {
+        ops = peak = 0;
+        ind_ = ind;
+        std::vector<Factor> fs;
+        for (int r = 0; r < n_; ++r) {
+            Factor f;
+            f.row = r;
+            for (int c = 0; c < m_; ++c)
+                if (b_[(size_t)r * n_ + c] != 0.0) f.scope.push_back(c);
+            if (!f.scope.empty()) fs.push_back(std::move(f));
+        }
+        std::vector<int> left(m_);
+        for (int c = 0; c < m_; ++c) left[c] = c;
+        while (!left.empty()) {
+            size_t pick = 0, least = 99;
+            for (size_t i = 0; i < left.size(); ++i) {  // the column whose rows tie the fewest others
+                std::vector<int> u;
+                for (const Factor& f : fs)
+                    if (has(f, left[i])) u = unite(u, f.scope);
+                if (u.empty()) return false;
+                if (u.size() < least) {
+                    least = u.size();
+                    pick = i;
+                }
+            }
+            const int c = left[pick];
+            left.erase(left.begin() + pick);
+            std::vector<Factor> with, rest;
+            for (Factor& f : fs) {
+                if (has(f, c)) write_row(f, ops);
+                (has(f, c) ? with : rest).push_back(std::move(f));
+            }
+            while (with.size() > 2) {  // the pair with the smallest common scope first
+                size_t bi = 1, bj = 0, bs = 99;
+                for (size_t i = 1; i < with.size(); ++i)
+                    for (size_t j = 0; j < i; ++j) {
+                        const size_t w = unite(with[i].scope, with[j].scope).size();
+                        if (w < bs) {
+                            bs = w;
+                            bi = i;
+                            bj = j;
+                        }
+                    }
+                Factor f = multiply(with[bj], with[bi], ops);
+                with.erase(with.begin() + bi);
+                with[bj] = std::move(f);
+            }
+            rest.push_back(sum_out(with, c, ops));
+            fs = std::move(rest);
+            int alive = 0;
+            for (const Factor& f : fs) alive += (f.pure ? 1 : 2) * (int)f.val.size();  // (unwritten rows: none)
+            peak = std::max(peak, alive);
+            if (peak > 1024) return false;
+        }
+        std::string P, A;
+        for (const Factor& f : fs) {
+            P += (P.empty() ? "" : " * ") + f.val[0];
+            A += (A.empty() ? "" : " * ") + f.abs[0];
+            ops += 2;
+        }
+        line("const double P = " + P + ", A = " + A + ";");
+        if (code) *code = out_.str();
+        return true;
+    }
+
+private:
+    static bool has(const Factor& f, int c) { return std::find(f.scope.begin(), f.scope.end(), c) != f.scope.end(); }
+    static std::vector<int> unite(const std::vector<int>& a, const std::vector<int>& b)
+    {
+        std::vector<int> u;
+        std::set_union(a.begin(), a.end(), b.begin(), b.end(), std::back_inserter(u));
+        return u;
+    }
+    // Index into f of the setting `i` over `scope` (a superset of f's).
+    static size_t project(const Factor& f, const std::vector<int>& scope, size_t i)
+    {
+        size_t k = 0;
+        for (size_t p = 0; p < f.scope.size(); ++p) {
+            const size_t at = std::lower_bound(scope.begin(), scope.end(), f.scope[p]) - scope.begin();
+            k |= ((i >> at) & 1u) << p;
+        }
+        return k;
+    }
+    void line(const std::string& t) { out_ << ind_ << t << "\n"; }
+    std::string fresh(const char* stem) { return stem + std::to_string(id_++); }
+    static std::string fabs(const std::string& v) { return "__builtin_fabs(" + v + ")"; }
+
+    void write_row(Factor& f, int& ops)
+    {
+        if (f.row < 0) return;
+        f.val.push_back("x" + std::to_string(f.row));
+        for (size_t k = 0; k < f.scope.size(); ++k)
+            for (size_t i = 0, end = size_t(1) << k; i < end; ++i) {
+                const std::string v = fresh("v");
+                line("const double " + v + " = " + f.val[i] + " + " + hexlit(b_[(size_t)f.row * n_ + f.scope[k]]) + ";");
+                f.val.push_back(v);
+                ++ops;
+            }
+        for (const std::string& v : f.val) f.abs.push_back(fabs(v));
+        f.row = -1;
+    }
+    Factor multiply(const Factor& f, const Factor& g, int& ops)
+    {
+        Factor h;
+        h.scope = unite(f.scope, g.scope);
+        h.pure = f.pure && g.pure;
+        for (size_t i = 0; i < size_t(1) << h.scope.size(); ++i) {
+            const size_t fi = project(f, h.scope, i), gi = project(g, h.scope, i);
+            const std::string v = fresh("p");
+            line("const double " + v + " = " + f.val[fi] + " * " + g.val[gi] + ";");
+            h.val.push_back(v);
+            ++ops;
+            if (h.pure) {
+                h.abs.push_back(fabs(v));
+            } else {
+                const std::string u = fresh("q");
+                line("const double " + u + " = " + f.abs[fi] + " * " + g.abs[gi] + ";");
+                h.abs.push_back(u);
+                ++ops;
+            }
+        }
+        return h;
+    }
+    Factor sum_out(const std::vector<Factor>& fs, int c, int& ops)
+    {
+        const std::vector<int> scope = fs.size() == 2 ? unite(fs[0].scope, fs[1].scope) : fs[0].scope;
+        const size_t at = std::lower_bound(scope.begin(), scope.end(), c) - scope.begin();
+        Factor h;
+        h.pure = false;
+        for (int s : scope)
+            if (s != c) h.scope.push_back(s);
+        for (size_t i = 0; i < size_t(1) << h.scope.size(); ++i) {
+            const size_t i0 = ((i >> at) << (at + 1)) | (i & ((size_t(1) << at) - 1)), i1 = i0 | (size_t(1) << at);
+            const std::string v = fresh("t"), u = fresh("u");
+            const Factor& f = fs[0];
+            const size_t f0 = project(f, scope, i0), f1 = project(f, scope, i1);
+            if (fs.size() == 1) {
+                line("const double " + v + " = " + f.val[f0] + " - " + f.val[f1] + ";");
+                line("const double " + u + " = " + f.abs[f0] + " + " + f.abs[f1] + ";");
+                ops += 2;
+            } else {
+                const Factor& g = fs[1];
+                const size_t g0 = project(g, scope, i0), g1 = project(g, scope, i1);
+                const std::string p = fresh("p");
+                line("const double " + p + " = " + f.val[f0] + " * " + g.val[g0] + ";");
+                line("const double " + v + " = __builtin_fma(-" + f.val[f1] + ", " + g.val[g1] + ", " + p + ");");
+                std::string q = fabs(p);
+                ops += 3;
+                if (!f.pure || !g.pure) {
+                    q = fresh("q");
+                    line("const double " + q + " = " + f.abs[f0] + " * " + g.abs[g0] + ";");
+                    ++ops;
+                }
+                line("const double " + u + " = __builtin_fma(" + f.abs[f1] + ", " + g.abs[g1] + ", " + q + ");");
+            }
+            h.val.push_back(v);
+            h.abs.push_back(u);
+        }
+        return h;
+    }
+
+    const std::vector<double>& b_;
+    int n_, m_;
+    const char* ind_ = "";
+    int id_ = 0;
+    std::ostringstream out_;
+};
+
 }  // namespace
+
+// The end of a real kernel: the chunk's sums into the lane's, and the block's
+// record.
+static void emit_real_tail(std::ostringstream& o)
+{
+    o << "        if (h < num_chunks) { ddadd(a_hi, a_lo, t_hi, t_lo); a_abs += t_abs; }\n"
+         "    }\n"
+         "    for (int off = 32; off >= 1; off >>= 1) {\n"
+         "        const double oh = __shfl_xor(a_hi, off, 64), ol = __shfl_xor(a_lo, off, 64);\n"
+         "        const double oa = __shfl_xor(a_abs, off, 64);\n"
+         "        ddadd(a_hi, a_lo, oh, ol);\n"
+         "        a_abs += oa;\n"
+         "    }\n"
+         "    const int w = threadIdx.x >> 6;\n"
+         "    if (lane == 0) { red[3 * w] = a_hi; red[3 * w + 1] = a_lo; red[3 * w + 2] = a_abs; }\n"
+         "    __syncthreads();\n"
+         "    if (threadIdx.x == 0) {\n"
+         "        double hh = red[0], ll = red[1], aa = red[2];\n"
+         "        for (int i = 1; i < 4; ++i) { ddadd(hh, ll, red[3 * i], red[3 * i + 1]); aa += red[3 * i + 2]; }\n"
+         "        double* out = partial + 4 * blockIdx.x;\n"
+         "        if (accumulate) { ddadd(hh, ll, out[0], out[1]); aa += out[2]; }\n"
+         "        out[0] = hh; out[1] = ll; out[2] = aa; out[3] = 0.0;\n"
+         "    }\n"
+         "}\n";
+}
+
+// The number m of inner columns to sum out: the least operations per subset
+// among those whose code stays within kElimOps instructions (compile time)
+// and whose tables within kElimPeak values, leaving at least 2^19 outer
+// settings to share out.  0: walk.  The kernels take up to 512 VGPRs, one
+// wave per SIMD: straight-line code has its own parallelism, and at two
+// waves (256 VGPRs) the larger ones spill (order 38, 7 per row 6.0 -> 7.4 ms,
+// at three 20 ms).  Kernel ms of the walk and at 700 operations with 64
+// values, then 1200 with 128, N(0,1) entries: order 36 with 5 per row 8.1,
+// 0.39, 0.32; order 38 with 7 42, 6.0, 2.7; order 40 with 8 215, 55.7, 53.9;
+// order 30 with 4 0.11, 0.013.  Below order 26 a walk takes 0.02 ms.
+int real_elim_columns(const double* b, int n)
+{
+    constexpr int kElimOps = 1000, kElimPeak = 128;
+    if (n < 26) return 0;
+    const std::vector<double> v(b, b + (size_t)n * n);
+    int best = 0;
+    double least = 1e300;
+    for (int m = 3; m <= std::min(16, n - 20); ++m) {
+        int ops = 0, peak = 0, outer = 0;
+        if (!Eliminator(v, n, m).run(ops, peak, nullptr, "") || ops > kElimOps || peak > kElimPeak) continue;
+        for (int r = 0; r < n; ++r) {
+            bool in = false;
+            for (int c = 0; c < m; ++c) in = in || b[(size_t)r * n + c] != 0.0;
+            outer += in ? 0 : 1;
+        }
+        const double cost = std::ldexp(ops + outer + 16.0, -m);
+        if (cost < least) {
+            least = cost;
+            best = m;
+        }
+    }
+    return least < 4.0 ? best : 0;  // the walk takes 4-10 instructions per subset
+}
+
+static std::string emit_real_elim_kernel(const std::vector<double>& b, int n, bool compensated,
+                                         const std::string& name, int m)
+{
+    std::vector<double> x0(n);
+    for (int i = 0; i < n; ++i) {  // as emit_real_kernel
+        double rs = 0.0;
+        for (int j = 0; j < n; ++j) rs += b[(size_t)i * n + j];
+        x0[i] = b[(size_t)i * n + n - 1] - rs / 2;
+    }
+    int ops = 0, peak = 0;
+    std::string inner;
+    Eliminator(b, n, m).run(ops, peak, &inner, "            ");
+    std::ostringstream o;
+    o << "// generated: SpaRyser kernel for one " << n << "x" << n << " real matrix (FP64, "
+      << (compensated ? "compensated" : "plain") << " sums, " << m << " inner columns summed out in " << ops
+      << " operations)\n";
+    o << "static __device__ __forceinline__ void ts(double a, double b, double& s, double& e)\n"
+         "{ s = a + b; const double bb = s - a; e = (a - (s - bb)) + (b - bb); }\n"
+         "static __device__ __forceinline__ void ddadd(double& ah, double& al, double bh, double bl)\n"
+         "{ double s, e; ts(ah, bh, s, e); e += al + bl; ah = s + e; al = e - (ah - s); }\n";
+    o << "extern \"C\" __global__ void __launch_bounds__(256)\n" << name
+      << "(double* __restrict__ partial, unsigned long long task_begin,\n"
+         "    unsigned long long task_end, unsigned long long num_chunks, int L, int accumulate)\n{\n";
+    o << "    __shared__ double red[12];\n"
+         "    const unsigned lane = threadIdx.x & 63u;\n"
+         "    const unsigned long long wave = (unsigned long long)blockIdx.x * 4 + (threadIdx.x >> 6);\n"
+         "    const unsigned long long nwave = (unsigned long long)gridDim.x * 4;\n"
+         "    const int Lo = L - " << m << ";  // a chunk's outer steps, over columns " << m << ".. in Gray order\n"
+         "    double a_hi = 0.0, a_lo = 0.0, a_abs = 0.0;\n"
+         "    for (unsigned long long task = task_begin + wave; task < task_end; task += nwave) {\n"
+         "        const unsigned long long h = task * 64 + lane;\n";
+    o << "        double ";
+    for (int i = 0; i < n; ++i) o << "x" << i << " = " << hexlit(x0[i]) << (i + 1 < n ? ", " : ";\n");
+    o << "        const unsigned long long k0 = h << Lo;\n"
+         "        const unsigned long long g0 = k0 ^ (k0 >> 1);\n";
+    for (int j = m; j < n - 1; ++j) {
+        bool any = false;
+        for (int r = 0; r < n; ++r) any = any || b[(size_t)r * n + j] != 0.0;
+        if (!any) continue;
+        o << "        { const double bj = ((((g0 >> " << j - m << ") & 1ull) != 0ull) && (" << j - m
+          << " >= Lo - 1)) ? 1.0 : 0.0;";
+        for (int r = 0; r < n; ++r) {
+            const double d = b[(size_t)r * n + j];
+            if (d != 0.0) o << " x" << r << " = __builtin_fma(bj, " << hexlit(d) << ", x" << r << ");";
+        }
+        o << " }\n";
+    }
+    o << "        const double sd = (h & 1ull) ? -1.0 : 1.0;  // direction of the last outer column\n"
+         "        double t_hi = 0.0, t_lo = 0.0, t_abs = 0.0, blk = 0.0, ba = 0.0;\n"
+         "        const unsigned steps = 1u << Lo, half = steps >> 1;\n"
+         "#pragma nounroll\n"
+         "        for (unsigned s = 0;;) {\n";
+    o << inner;
+    std::vector<std::string> chain(4);
+    int k = 0;
+    for (int r = 0; r < n; ++r) {
+        bool in = false;
+        for (int c = 0; c < m; ++c) in = in || b[(size_t)r * n + c] != 0.0;
+        if (in) continue;
+        std::string& c = chain[k++ % 4];
+        c += (c.empty() ? "x" : " * x") + std::to_string(r);
+    }
+    std::string prod;
+    for (const std::string& c : chain)
+        if (!c.empty()) prod += (prod.empty() ? "(" : " * (") + c + ")";
+    o << "            const double S = " << (prod.empty() ? "1.0" : prod) << ";\n"
+         "            blk = __builtin_fma((s & 1u) ? -P : P, S, blk);\n"
+         "            ba = __builtin_fma(A, __builtin_fabs(S), ba);\n"
+         "            ++s;\n"
+         "            if ((s & 3u) == 0u || s == steps) "
+      << (compensated ? "{ double s_, e_; ts(t_hi, blk, s_, e_); t_hi = s_; t_lo += e_; t_abs += ba; blk = 0.0; ba = 0.0; }\n"
+                      : "{ t_hi += blk; t_abs += ba; blk = 0.0; ba = 0.0; }\n")
+      << "            if (s == steps) break;\n"
+         "            const double sdm = (s == half) ? sd : (((s >> (__builtin_ctz(s) + 1)) & 1u) ? -1.0 : 1.0);\n";
+    for (int c = m; c < n - 1 && c - m < 16; ++c) {
+        o << "            " << (c == m ? "if" : "} else if") << " (s & " << (1u << (c - m)) << "u) {\n";
+        emit_real_flip(o, b, n, c, 0, "                ", "sdm");
+    }
+    o << "            }\n"
+         "        }\n";
+    emit_real_tail(o);
+    return o.str();
+}
 
 std::string emit_real_kernel(const std::vector<double>& b, int n, bool compensated, const std::string& name)
 {
+    if (const int m = real_elim_columns(b.data(), n)) return emit_real_elim_kernel(b, n, compensated, name, m);
     const int U = gen_unroll_bits_real(n);
     const RealLevels lv = real_levels(b, n);
     std::vector<double> x0(n);
@@ -717,25 +1058,7 @@ std::string emit_real_kernel(const std::vector<double>& b, int n, bool compensat
     emit_real_term(o, lv, false, "            ");
     block_tail("            ");
     o << "        }\n";
-    o << "        if (h < num_chunks) { ddadd(a_hi, a_lo, t_hi, t_lo); a_abs += t_abs; }\n"
-         "    }\n"
-         "    for (int off = 32; off >= 1; off >>= 1) {\n"
-         "        const double oh = __shfl_xor(a_hi, off, 64), ol = __shfl_xor(a_lo, off, 64);\n"
-         "        const double oa = __shfl_xor(a_abs, off, 64);\n"
-         "        ddadd(a_hi, a_lo, oh, ol);\n"
-         "        a_abs += oa;\n"
-         "    }\n"
-         "    const int w = threadIdx.x >> 6;\n"
-         "    if (lane == 0) { red[3 * w] = a_hi; red[3 * w + 1] = a_lo; red[3 * w + 2] = a_abs; }\n"
-         "    __syncthreads();\n"
-         "    if (threadIdx.x == 0) {\n"
-         "        double hh = red[0], ll = red[1], aa = red[2];\n"
-         "        for (int i = 1; i < 4; ++i) { ddadd(hh, ll, red[3 * i], red[3 * i + 1]); aa += red[3 * i + 2]; }\n"
-         "        double* out = partial + 4 * blockIdx.x;\n"
-         "        if (accumulate) { ddadd(hh, ll, out[0], out[1]); aa += out[2]; }\n"
-         "        out[0] = hh; out[1] = ll; out[2] = aa; out[3] = 0.0;\n"
-         "    }\n"
-         "}\n";
+    emit_real_tail(o);
     return o.str();
 }
 

@@ -137,6 +137,8 @@ constexpr int kGenPruneChunk = 5;
 constexpr int kGenPruneUnroll = 2;
 bool gen_pruned(const int64_t* b, int n);
 int codegen_real_unroll_bits(int n);
+// Inner columns a real kernel sums out of a chunk in one go (0: it walks).
+int real_elim_columns(const double* b, int n);
 uint64_t pattern_hash(const int64_t* b, int n, int options);
 int codegen_get_kernel(int device, uint64_t hash, const std::string& src, const std::string& name, hipFunction_t* fn,
                        double* compile_s, bool* cached);
