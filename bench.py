@@ -22,10 +22,10 @@ mostly per-call cost; and `secondary` -- the dense n=24, sparse 0/1 n=40
 with inputs resident.
 
 roofline.achieved counts the algorithmic 2n FP64 flops per subset (n adds +
-n-1 multiplies + 1 accumulate) over the kernel's duration measured with HIP
-events on its own stream; peak = MI355X FP64 vector; ceiling = the issue
-ceiling 2n/(2(2n-1)) of peak of any Gray-code Ryser (2n-1 FP64 instructions
-per subset).
+n-1 multiplies + 1 accumulate) over the kernel's duration by the device's
+clock; peak = MI355X FP64 vector; ceiling = the issue ceiling 2n/(3n+3) of
+peak of a Gray-code Ryser that takes two subsets per step (3n+3 FP64
+instructions for two).
 cpu_baseline = the reference's CPU Gray-code walk (restated in oracle/, same
 chunking and arithmetic order) on a bounded sample of the same walk, timed
 on this host's cores and scaled to permanents per second.
@@ -458,11 +458,12 @@ def main(argv=None):
     flops = 2.0 * n * float(1 << (n - 1))  # algorithmic 2n flops per subset
     k_ms = float(np.mean(kernel_ms))
     achieved = flops / (k_ms * 1e-3) / 1e12
-    # Issue ceiling of any Gray-code Ryser under the 2n convention: at least
-    # 2n-1 FP64 VALU instructions per subset (n adds, n-2 multiplies, one
-    # FMA into the sum); the peak counts 2 flops (an FMA) per instruction
-    # slot, so 2n algorithmic flops in 2n-1 slots reach 2n/(2(2n-1)) of it.
-    ceiling = PEAK_FP64_TFLOPS * (2.0 * n) / (2.0 * (2.0 * n - 1.0))
+    # Issue ceiling under the 2n convention: for two subsets n adds, two
+    # products of n - 1 rows (n - 2 multiplies; 4 adds that start the chains
+    # and n - 2 multiplies or FMAs) and 3 instructions into the sum are 3n + 3;
+    # the peak counts 2 flops (an FMA) per instruction slot, so 4n algorithmic
+    # flops in 3n + 3 slots reach 4n/(2(3n + 3)) of it.
+    ceiling = PEAK_FP64_TFLOPS * (4.0 * n) / (2.0 * (3.0 * n + 3.0))
     out = {
         "metric": METRIC,
         "value": 1e3 / ms_per_step,
@@ -483,9 +484,9 @@ def main(argv=None):
         "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP64_TFLOPS, "traffic": measured_traffic(info["kernel"]),
                      "ceiling": ceiling, "frac_of_ceiling": achieved / ceiling,
-                     "ceiling_rule": "2n-1 FP64 VALU instructions per subset (n adds, n-2 multiplies, 1 FMA) at "
-                                     "the peak's issue rate: 2n/(2(2n-1)) of peak; >= 60% of peak is out of reach "
-                                     "for any Gray-code Ryser under the 2n-flop convention",
+                     "ceiling_rule": "3n+3 FP64 VALU instructions per two subsets (n adds, 2(n-2) multiplies and "
+                                     "FMAs, 4 chain starts, 3 into the sum) at the peak's issue rate: 2n/(3n+3) of "
+                                     "peak under the 2n-flop convention",
                      "kernel": info["kernel"], "kernel_ms": k_ms,
                      "flops_per_launch": flops, "flop_convention": "2n per subset (add, mul, accumulate; FMA = 2)",
                      "counters": measured_counters(info["kernel"], k_ms)},

@@ -70,7 +70,7 @@ typedef struct spm_result {
     int32_t is_exact;
     int32_t status;
     double seconds;       /* host wall time of the call                     */
-    double kernel_ms;     /* device time of the permanent kernels (events)  */
+    double kernel_ms;     /* device time of the permanent kernels, by its clock */
     uint64_t subsets;     /* 2^(n-1) Gray-code subsets walked               */
     int32_t n;
     int32_t launches;

@@ -49,7 +49,9 @@ SOURCES = [  # the longest compiles first, so that the job pool starts them earl
     ("int_sparse.hip", []),
     ("int_small.hip", []),
     ("int_prune.hip", []),
+    ("run_io.hip", []),
     ("prune.cpp", []),
+    ("workspace.cpp", []),
     ("batch_engine.cpp", []),
     ("decompose.cpp", []),
     ("codegen.cpp", []),

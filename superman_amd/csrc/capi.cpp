@@ -8,10 +8,12 @@
 
 #include "spm_host.h"
 #include "spm_kernels.h"
+#include "workspace.h"
 
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -59,6 +61,18 @@ int device_cus(int device, int* cus)
     g_cus[device] = v;
     *cus = v;
     return SPM_OK;
+}
+
+// The rate of the counter behind RunResult::ticks.
+static int device_clock_khz(int device)
+{
+    static std::atomic<int> khz[64];
+    if (device < 0 || device >= 64) return 100000;
+    int v = khz[device].load(std::memory_order_relaxed);
+    if (v > 0) return v;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeWallClockRate, device) != hipSuccess || v <= 0) v = 100000;
+    khz[device].store(v, std::memory_order_relaxed);
+    return v;
 }
 
 int blocks_per_cu(int device, const void* kern, int block, int* bpc, int lds_bytes)
@@ -170,24 +184,32 @@ struct spm_plan {
     uint64_t chunks = 0, tasks = 0;
     int slices = 1;
     int max_grid = 0;      // resident blocks on the device (dense kinds)
-    int partial_cap = 0;   // per-block records allocated in d_partial
     int rec = 4;    // doubles per per-block partial record
     int comps = 1;  // double-double components per record (1 real, 2 complex)
     const void* kern = nullptr;
+    // Memory, all in one workspace: the matrix and x(empty set) (staged in
+    // h_M, h_x0 until the first run's begin kernel copies them), the
+    // per-block records and what the pruned walk needs.
+    Workspace* ws = nullptr;
+    size_t in_bytes = 0;     // staged bytes
+    bool uploaded = false;
+    bool busy = false;       // a run was started and has not returned its result
     double* d_M = nullptr;   // dense kinds; the integer kind stores int32 here
     double* d_x0 = nullptr;
+    char* h_M = nullptr;
+    char* h_x0 = nullptr;
+    unsigned long long* d_t0 = nullptr;  // the run's start time
+    size_t counter_bytes = 0;            // zeroed at the start of every run
     double log2_bound = 0;   // integer kind: log2 of the bound on |T|
     int halved = 0;          // integer kinds: rows carried halved (int_row_weights)
     bool pair = false;       // dense real plans: the matrix is scaled for dense_pair_kernel
     PairScale scale;
     int log2_scale = 0;      // FP32-product plans: perm = 2^log2_scale perm(scaled)
     double* d_partial = nullptr;
-    double* d_out = nullptr;
-    double* h_out = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    int records = 0;         // per-block records of a run
     int block = kDenseBlock;
     int lds_bytes = 0;       // integer kind, pruned walk: dynamic LDS
-    unsigned int* d_counter = nullptr;  // its counters, a set per launch (0 between runs)
+    unsigned int* d_counter = nullptr;  // its counters, a set per launch
     unsigned long long* d_list[2] = {nullptr, nullptr};
     unsigned int list_cap = 0;          // prefixes per list segment
     int first_group = 0;                // PrunePlan::first_group
@@ -203,27 +225,113 @@ struct spm_plan {
 static void plan_free(spm_plan* p)
 {
     if (!p) return;
-    DeviceGuard g(p->device);
-    if (p->d_M) (void)hipFree(p->d_M);
-    if (p->d_x0) (void)hipFree(p->d_x0);
-    if (p->d_partial) (void)hipFree(p->d_partial);
-    if (p->d_counter) (void)hipFree(p->d_counter);
-    for (unsigned long long* l : p->d_list)
-        if (l) (void)hipFree(l);
-    if (p->d_out) (void)hipFree(p->d_out);
-    if (p->h_out) (void)hipHostFree(p->h_out);
-    if (p->ev0) (void)hipEventDestroy(p->ev0);
-    if (p->ev1) (void)hipEventDestroy(p->ev1);
+    if (p->ws) workspace_put(p->ws, !p->busy);
     delete p;
 }
 
-#define SPM_TRY(expr)                                  \
-    do {                                               \
-        if ((expr) != hipSuccess) {                    \
-            plan_free(p);                              \
-            return SPM_EHIP;                           \
-        }                                              \
-    } while (0)
+// A plan's workspace, split into its arrays (256-byte aligned).
+static int plan_memory(spm_plan* p, size_t m_bytes, size_t x0_bytes, size_t partial_bytes, size_t counter_bytes = 0,
+                       size_t list_bytes = 0)
+{
+    auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+    p->in_bytes = up(m_bytes) + up(x0_bytes);
+    p->counter_bytes = up(counter_bytes);
+    size_t off = p->in_bytes;
+    const size_t partial = off;
+    off += up(partial_bytes);
+    const size_t counter = off;
+    off += p->counter_bytes;
+    const size_t t0 = off;
+    off += 256;
+    const size_t list = off;
+    off += 2 * up(list_bytes);
+    const int rc = workspace_get(p->device, off, p->in_bytes, &p->ws);
+    if (rc != SPM_OK) return rc;
+    char* d = p->ws->dev;
+    p->d_M = (double*)d;
+    p->d_x0 = (double*)(d + up(m_bytes));
+    p->h_M = p->ws->host;
+    p->h_x0 = p->ws->host + up(m_bytes);
+    p->d_partial = (double*)(d + partial);
+    p->d_t0 = (unsigned long long*)(d + t0);
+    if (counter_bytes) p->d_counter = (unsigned int*)(d + counter);
+    if (list_bytes) {
+        p->d_list[0] = (unsigned long long*)(d + list);
+        p->d_list[1] = (unsigned long long*)(d + list + up(list_bytes));
+    }
+    p->uploaded = p->in_bytes == 0;
+    return SPM_OK;
+}
+
+// The first kernel of a run: uploads what is staged, zeroes the counters and
+// notes the start time.
+static int run_begin(spm_plan* p, hipStream_t st)
+{
+    const char* src = p->ws->host_dev;
+    unsigned int words = p->uploaded ? 0u : (unsigned int)(p->in_bytes / 16);
+    unsigned int zwords = (unsigned int)(p->counter_bytes / 16);
+    const unsigned int blocks = std::min(32u, std::max(1u, (std::max(words, zwords) + 255) / 256));
+    void* args[] = {&src, &p->d_M, &words, &p->d_counter, &zwords, &p->d_t0};
+    p->busy = true;
+    if (hipLaunchKernel(run_begin_kernel_ptr(), dim3(blocks), dim3(256), args, 0, st) != hipSuccess) return SPM_EHIP;
+    p->uploaded = true;
+    return SPM_OK;
+}
+
+// Waits for the run's flag: by polling while the run is short (a stream
+// synchronization costs 5 us more), then through the stream, whose error is
+// the run's.
+static int run_wait(spm_plan* p, hipStream_t st)
+{
+    const unsigned int seq = p->ws->seq;
+    auto arrived = [&] { return __atomic_load_n(&p->ws->result_host->flag, __ATOMIC_ACQUIRE) == seq; };
+    constexpr double kPoll = 200e-6, kLate = 2.0;
+    auto poll = [&](double limit) {
+        const double t0 = now_seconds();
+        do {
+            for (int i = 0; i < 64; ++i) {
+                if (arrived()) return true;
+                __builtin_ia32_pause();
+            }
+        } while (now_seconds() - t0 < limit);
+        return false;
+    };
+    if (!poll(kPoll)) {
+        if (hipStreamSynchronize(st) != hipSuccess) return SPM_EHIP;
+        if (!poll(kLate)) return SPM_EHIP;
+    }
+    p->busy = false;
+    return SPM_OK;
+}
+
+static double run_ms(spm_plan* p)
+{
+    return (double)p->ws->result_host->ticks / (double)device_clock_khz(p->device);
+}
+
+// Uploads a plan that outlives the call that made it.
+static int plan_upload(spm_plan* p)
+{
+    if (p->uploaded) return SPM_OK;
+    DeviceGuard guard(p->device);
+    if (!guard.ok()) return SPM_EHIP;
+    const int rc = run_begin(p, nullptr);
+    if (rc != SPM_OK || hipStreamSynchronize(nullptr) != hipSuccess) return SPM_EHIP;
+    p->busy = false;
+    return SPM_OK;
+}
+
+// spm_plan_*: a made plan, uploaded.
+static int finish_plan(int rc, spm_plan** out)
+{
+    if (rc != SPM_OK) return rc;
+    rc = plan_upload(*out);
+    if (rc != SPM_OK) {
+        plan_free(*out);
+        *out = nullptr;
+    }
+    return rc;
+}
 
 // Grid and launch slices of a dense plan for its geometry (L, tasks): as many
 // blocks as the tasks fill, at most the resident ones; very long runs
@@ -313,22 +421,16 @@ static int make_dense_plan(int kind, const double* a, int n, int precision, int 
     // Host preparation (dpSingleGPU.cuh:62-82; gpuComputeComplex.cu:212-241).
     const size_t col = (size_t)w * n;   // doubles per column
     const size_t plane = col * n;
-    std::vector<double> colmaj(2 * plane), x0(col);
     if (f32p) {
         p->log2_scale = f32prod_scale(a, n, scaled.data());
         a = scaled.data();
     }
-    dense_prepare(a, n, w, colmaj.data(), x0.data());
-    SPM_TRY(hipMalloc(&p->d_M, sizeof(double) * 2 * plane));
-    SPM_TRY(hipMalloc(&p->d_x0, sizeof(double) * col));
-    SPM_TRY(hipMalloc(&p->d_partial, sizeof(double) * p->rec * p->grid));
-    p->partial_cap = p->grid;
-    SPM_TRY(hipMalloc(&p->d_out, sizeof(double) * 6));
-    SPM_TRY(hipHostMalloc(&p->h_out, sizeof(double) * 6, hipHostMallocDefault));
-    SPM_TRY(hipMemcpy(p->d_M, colmaj.data(), sizeof(double) * 2 * plane, hipMemcpyHostToDevice));
-    SPM_TRY(hipMemcpy(p->d_x0, x0.data(), sizeof(double) * col, hipMemcpyHostToDevice));
-    SPM_TRY(hipEventCreate(&p->ev0));
-    SPM_TRY(hipEventCreate(&p->ev1));
+    if (plan_memory(p, sizeof(double) * 2 * plane, sizeof(double) * col, sizeof(double) * p->rec * p->max_grid) !=
+        SPM_OK) {
+        plan_free(p);
+        return SPM_EHIP;
+    }
+    dense_prepare(a, n, w, (double*)p->h_M, (double*)p->h_x0);
     *out = p;
     return SPM_OK;
 }
@@ -385,29 +487,18 @@ static int make_prune_plan(const PrunePlan& pr, int n, double log2_bound, int ha
         // and prefixes past 2^22 (2 x 42 MB) are walked where they are found.
         const double cap = std::min(64.0 * std::max(pr.nodes, pr.upper), std::ldexp(1.0, std::min(22, n - 13)));
         p->list_cap = (unsigned)std::max(512.0, std::ceil(cap * 1.25 / kPruneSets));
-        for (unsigned long long*& l : p->d_list)
-            if (hipMalloc(&l, sizeof(unsigned long long) * p->list_cap * kPruneSets) != hipSuccess) {
-                (void)hipGetLastError();
-                l = nullptr;
-                plan_free(p);
-                return SPM_ENOMEM;
-            }
     }
     char kn[96];
     std::snprintf(kn, sizeof kn, "int_prune_kernel<%d, %d>", pr.field_bytes, pr.dwords);
     p->kname = kn;
-    SPM_TRY(hipMalloc(&p->d_M, sizeof(int) * pr.blob.size()));
-    SPM_TRY(hipMemcpy(p->d_M, pr.blob.data(), sizeof(int) * pr.blob.size(), hipMemcpyHostToDevice));
-    const int records = p->grid * (p->first_group - 2) + p->grid2;  // a record per block and launch
-    const size_t counters = sizeof(unsigned int) * kPruneSets * kPruneCounterStride * p->first_group;
-    SPM_TRY(hipMalloc(&p->d_counter, counters));
-    SPM_TRY(hipMemset(p->d_counter, 0, counters));
-    SPM_TRY(hipMalloc(&p->d_partial, sizeof(unsigned long long) * 2 * records));
-    p->partial_cap = records;
-    SPM_TRY(hipMalloc(&p->d_out, sizeof(double) * 6));
-    SPM_TRY(hipHostMalloc(&p->h_out, sizeof(double) * 6, hipHostMallocDefault));
-    SPM_TRY(hipEventCreate(&p->ev0));
-    SPM_TRY(hipEventCreate(&p->ev1));
+    p->records = p->grid * (p->first_group - 2) + p->grid2;  // a record per block and launch
+    if (plan_memory(p, sizeof(int) * pr.blob.size(), 0, sizeof(unsigned long long) * 2 * p->records,
+                    sizeof(unsigned int) * kPruneSets * kPruneCounterStride * p->first_group,
+                    sizeof(unsigned long long) * p->list_cap * kPruneSets) != SPM_OK) {
+        plan_free(p);
+        return SPM_ENOMEM;
+    }
+    std::memcpy(p->h_M, pr.blob.data(), sizeof(int) * pr.blob.size());
     *out = p;
     return SPM_OK;
 }
@@ -492,52 +583,43 @@ static int make_int_plan(const int64_t* a, int n, int walk, int device, spm_plan
                   n);
     p->kname = kn;
     const size_t nn = (size_t)n * n;
-    if (sp) {
-        std::vector<int> blob;
-        int_sparse_blob(a, n, blob, w.data());
-        SPM_TRY(hipMalloc(&p->d_M, sizeof(int) * blob.size()));
-        std::vector<int> ys(y0.begin(), y0.end());
-        ys.push_back(small ? 1 : 0);  // products in FP64 groups (int_sparse_kernel)
-        SPM_TRY(hipMalloc(&p->d_x0, sizeof(int) * ys.size()));
-        SPM_TRY(hipMemcpy(p->d_M, blob.data(), sizeof(int) * blob.size(), hipMemcpyHostToDevice));
-        SPM_TRY(hipMemcpy(p->d_x0, ys.data(), sizeof(int) * ys.size(), hipMemcpyHostToDevice));
-    } else if (fp) {
-        std::vector<double> colmaj(2 * nn), yd(y0.begin(), y0.end());
-        int_small_planes(a, n, colmaj.data(), w.data());
-        SPM_TRY(hipMalloc(&p->d_M, sizeof(double) * 2 * nn));
-        SPM_TRY(hipMalloc(&p->d_x0, sizeof(double) * n));
-        SPM_TRY(hipMemcpy(p->d_M, colmaj.data(), sizeof(double) * 2 * nn, hipMemcpyHostToDevice));
-        SPM_TRY(hipMemcpy(p->d_x0, yd.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-    } else {
-        std::vector<int> colmaj(2 * nn);
-        int_planes(a, n, colmaj.data(), w.data());
-        SPM_TRY(hipMalloc(&p->d_M, sizeof(int) * 2 * nn));
-        SPM_TRY(hipMalloc(&p->d_x0, sizeof(int) * n));
-        SPM_TRY(hipMemcpy(p->d_M, colmaj.data(), sizeof(int) * 2 * nn, hipMemcpyHostToDevice));
-        SPM_TRY(hipMemcpy(p->d_x0, y0.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+    std::vector<int> blob;
+    if (sp) int_sparse_blob(a, n, blob, w.data());
+    p->records = p->grid;
+    if (plan_memory(p, sp ? sizeof(int) * blob.size() : (fp ? sizeof(double) : sizeof(int)) * 2 * nn,
+                    fp ? sizeof(double) * n : sizeof(int) * (n + 1), sizeof(unsigned long long) * 2 * p->grid) !=
+        SPM_OK) {
+        plan_free(p);
+        return SPM_EHIP;
     }
-    SPM_TRY(hipMalloc(&p->d_partial, sizeof(unsigned long long) * 2 * p->grid));
-    SPM_TRY(hipMalloc(&p->d_out, sizeof(double) * 6));
-    SPM_TRY(hipHostMalloc(&p->h_out, sizeof(double) * 6, hipHostMallocDefault));
-    SPM_TRY(hipEventCreate(&p->ev0));
-    SPM_TRY(hipEventCreate(&p->ev1));
+    if (sp) {
+        std::memcpy(p->h_M, blob.data(), sizeof(int) * blob.size());
+        std::memcpy(p->h_x0, y0.data(), sizeof(int) * n);
+        ((int*)p->h_x0)[n] = small ? 1 : 0;  // products in FP64 groups (int_sparse_kernel)
+    } else if (fp) {
+        int_small_planes(a, n, (double*)p->h_M, w.data());
+        for (int i = 0; i < n; ++i) ((double*)p->h_x0)[i] = y0[i];
+    } else {
+        int_planes(a, n, (int*)p->h_M, w.data());
+        std::memcpy(p->h_x0, y0.data(), sizeof(int) * n);
+    }
     *out = p;
     return SPM_OK;
 }
 
 extern "C" int spm_plan_dense_f64(const double* a, int n, int precision, int device, spm_plan** out)
 {
-    return make_dense_plan(1, a, n, precision, device, out);
+    return finish_plan(make_dense_plan(1, a, n, precision, device, out), out);
 }
 
 extern "C" int spm_plan_int(const int64_t* a, int n, int device, spm_plan** out)
 {
-    return make_int_plan(a, n, SPM_INT_WALK_AUTO, device, out);
+    return finish_plan(make_int_plan(a, n, SPM_INT_WALK_AUTO, device, out), out);
 }
 
 extern "C" int spm_plan_int_walk(const int64_t* a, int n, int walk, int device, spm_plan** out)
 {
-    return make_int_plan(a, n, walk, device, out);
+    return finish_plan(make_int_plan(a, n, walk, device, out), out);
 }
 
 // Generated SpaRyser plans (kind 4).
@@ -651,11 +733,11 @@ extern "C" int spm_plan_codegen(const int64_t* a, int n, int options, int device
         p->slices = 1;
         while (p->slices < est_s / 400.0 && p->slices < 1 << 12) p->slices *= 2;
     }
-    SPM_TRY(hipMalloc(&p->d_partial, sizeof(unsigned long long) * 2 * p->grid));
-    SPM_TRY(hipMalloc(&p->d_out, sizeof(double) * 6));
-    SPM_TRY(hipHostMalloc(&p->h_out, sizeof(double) * 6, hipHostMallocDefault));
-    SPM_TRY(hipEventCreate(&p->ev0));
-    SPM_TRY(hipEventCreate(&p->ev1));
+    p->records = p->grid;
+    if (plan_memory(p, 0, 0, sizeof(unsigned long long) * 2 * p->grid) != SPM_OK) {
+        plan_free(p);
+        return SPM_EHIP;
+    }
     *out = p;
     return SPM_OK;
 }
@@ -756,12 +838,10 @@ extern "C" int spm_plan_codegen_real(const double* a, int n, int options, int pr
     }
     p->max_grid = bpc * cus;
     dense_grid(p);
-    SPM_TRY(hipMalloc(&p->d_partial, sizeof(double) * p->rec * p->grid));
-    p->partial_cap = p->grid;
-    SPM_TRY(hipMalloc(&p->d_out, sizeof(double) * 6));
-    SPM_TRY(hipHostMalloc(&p->h_out, sizeof(double) * 6, hipHostMallocDefault));
-    SPM_TRY(hipEventCreate(&p->ev0));
-    SPM_TRY(hipEventCreate(&p->ev1));
+    if (plan_memory(p, 0, 0, sizeof(double) * p->rec * p->max_grid) != SPM_OK) {
+        plan_free(p);
+        return SPM_EHIP;
+    }
     *out = p;
     return SPM_OK;
 }
@@ -777,17 +857,17 @@ extern "C" int spm_plan_codegen_info(const spm_plan* p, double* compile_seconds,
 
 extern "C" int spm_plan_dense_c128(const double* a, int n, int precision, int device, spm_plan** out)
 {
-    return make_dense_plan(2, a, n, precision, device, out);
+    return finish_plan(make_dense_plan(2, a, n, precision, device, out), out);
 }
 
-#undef SPM_TRY
 
 static int dense_run(spm_plan* p, hipStream_t st, spm_result* r)
 {
     const double t0 = now_seconds();
     DeviceGuard guard(p->device);
     if (!guard.ok()) return SPM_EHIP;
-    if (hipEventRecord(p->ev0, st) != hipSuccess) return SPM_EHIP;
+    int rc = run_begin(p, st);
+    if (rc != SPM_OK) return rc;
     const uint64_t per = (p->tasks + p->slices - 1) / p->slices;
     int launches = 0;
     for (int s = 0; s < p->slices; ++s) {
@@ -807,24 +887,22 @@ static int dense_run(spm_plan* p, hipStream_t st, spm_result* r)
     }
     {
         int nrec = p->grid, stride = p->rec, comps = p->comps;
-        void* args[] = {&p->d_partial, &nrec, &stride, &comps, &p->d_out};
-        if (hipLaunchKernel(reduce_partials_kernel_ptr(), dim3(1), dim3(256), args, 0, st) != hipSuccess)
-            return SPM_EHIP;
+        unsigned int seq = ++p->ws->seq;
+        void* args[] = {&p->d_partial, &nrec, &stride, &comps, &p->d_t0, &p->ws->result, &seq};
+        if (hipLaunchKernel(run_end_dd_kernel_ptr(), dim3(1), dim3(256), args, 0, st) != hipSuccess) return SPM_EHIP;
     }
-    if (hipEventRecord(p->ev1, st) != hipSuccess) return SPM_EHIP;
-    if (hipMemcpyAsync(p->h_out, p->d_out, sizeof(double) * 3 * p->comps, hipMemcpyDeviceToHost, st) != hipSuccess)
-        return SPM_EHIP;
-    if (hipStreamSynchronize(st) != hipSuccess) return SPM_EHIP;
-    float ms = 0.f;
-    if (hipEventElapsedTime(&ms, p->ev0, p->ev1) != hipSuccess) ms = -1.f;
+    rc = run_wait(p, st);
+    if (rc != SPM_OK) return rc;
+    double rec[6];
+    std::memcpy(rec, p->ws->result_host->word, sizeof rec);
 
     std::memset(r, 0, sizeof *r);
     const int n = p->n;
-    if (p->pair) pair_finish(p->scale, p->h_out);
-    dense_fill_result(n, p->comps == 2, p->precision != SPM_PREC_PLAIN, p->h_out, r);
+    if (p->pair) pair_finish(p->scale, rec);
+    dense_fill_result(n, p->comps == 2, p->precision != SPM_PREC_PLAIN, rec, r);
     if (p->precision == SPM_PREC_F32_PRODUCT) f32prod_finish(n, p->log2_scale, r);
     r->status = SPM_OK;
-    r->kernel_ms = ms;
+    r->kernel_ms = run_ms(p);
     r->subsets = uint64_t(1) << (n - 1);
     r->n = n;
     r->launches = launches;
@@ -859,7 +937,8 @@ static int int_run(spm_plan* p, hipStream_t st, spm_result* r)
     const double t0 = now_seconds();
     DeviceGuard guard(p->device);
     if (!guard.ok()) return SPM_EHIP;
-    if (hipEventRecord(p->ev0, st) != hipSuccess) return SPM_EHIP;
+    int rc = run_begin(p, st);
+    if (rc != SPM_OK) return rc;
     const uint64_t per = (p->tasks + p->slices - 1) / p->slices;
     int launches = 0;
     for (int s = 0; s < p->slices; ++s) {
@@ -867,7 +946,7 @@ static int int_run(spm_plan* p, hipStream_t st, spm_result* r)
         if (tb >= te) break;
         int acc = s > 0 ? 1 : 0;
         if (p->d_counter) {
-            const int rc = prune_launch(p, tb, te, st);
+            rc = prune_launch(p, tb, te, st);
             if (rc != SPM_OK) return rc;
         } else if (p->kind == 4) {
             void* args[] = {&p->d_partial, &tb, &te, &p->chunks, &p->L, &acc};
@@ -881,23 +960,19 @@ static int int_run(spm_plan* p, hipStream_t st, spm_result* r)
         ++launches;
     }
     {
-        int nrec = p->d_counter ? p->partial_cap : p->grid, counters = kPruneSets * p->first_group;
-        void* args[] = {&p->d_partial, &nrec, &p->d_out, &p->d_counter, &counters};
-        const void* k = p->d_counter ? reduce_prune_kernel_ptr() : reduce_i128_kernel_ptr();
-        if (hipLaunchKernel(k, dim3(1), dim3(256), args, 0, st) != hipSuccess) return SPM_EHIP;
+        unsigned int seq = ++p->ws->seq;
+        void* args[] = {&p->d_partial, &p->records, &p->d_t0, &p->ws->result, &seq};
+        if (hipLaunchKernel(run_end_i128_kernel_ptr(), dim3(1), dim3(256), args, 0, st) != hipSuccess) return SPM_EHIP;
     }
-    if (hipEventRecord(p->ev1, st) != hipSuccess) return SPM_EHIP;
-    if (hipMemcpyAsync(p->h_out, p->d_out, 16, hipMemcpyDeviceToHost, st) != hipSuccess) return SPM_EHIP;
-    if (hipStreamSynchronize(st) != hipSuccess) return SPM_EHIP;
-    float ms = 0.f;
-    if (hipEventElapsedTime(&ms, p->ev0, p->ev1) != hipSuccess) ms = -1.f;
+    rc = run_wait(p, st);
+    if (rc != SPM_OK) return rc;
     std::memset(r, 0, sizeof *r);
     unsigned long long w[2];
-    std::memcpy(w, p->h_out, 16);
-    const int rc = int_fill_result(p->n, w[0], w[1], r, p->halved);
+    std::memcpy(w, p->ws->result_host->word, 16);
+    rc = int_fill_result(p->n, w[0], w[1], r, p->halved);
     if (rc != SPM_OK) return rc;
     r->status = SPM_OK;
-    r->kernel_ms = ms;
+    r->kernel_ms = run_ms(p);
     r->subsets = uint64_t(1) << (p->n - 1);
     r->n = p->n;
     r->launches = launches;
@@ -947,15 +1022,6 @@ extern "C" int spm_plan_set_log2_chunk(spm_plan* p, int L)
     p->chunks = uint64_t(1) << (B - L);
     p->tasks = (p->chunks + kWaveLanes - 1) / kWaveLanes;
     dense_grid(p);
-    if (p->grid > p->partial_cap) {
-        DeviceGuard guard(p->device);
-        if (!guard.ok()) return SPM_EHIP;
-        double* np = nullptr;
-        if (hipMalloc(&np, sizeof(double) * p->rec * p->grid) != hipSuccess) return SPM_ENOMEM;
-        if (p->d_partial) (void)hipFree(p->d_partial);
-        p->d_partial = np;
-        p->partial_cap = p->grid;
-    }
     return SPM_OK;
 }
 

@@ -5,9 +5,10 @@
 // xRegisterMSharedKahan and their placement variants).  The per-chunk walk is
 // in walk_f64.h, the grid-strided task loop and the block reduction in
 // dense_chunks.h; this file holds the kernels that take a matrix as it is
-// (those with a column to scale to ones are dense_pair.hip's) and the final
-// reduction kernel.
+// (those with a column to scale to ones are dense_pair.hip's) and a final
+// reduction kernel for spm_dense_f64_noalloc.
 #include "dense_chunks.h"
+#include "dense_reduce.h"
 
 namespace spm {
 
@@ -39,21 +40,10 @@ reduce_partials_kernel(const double* __restrict__ partial, int nrec, int stride,
                        double* __restrict__ out)
 {
     __shared__ double red[3 * (256 / kWave)];
-    for (int q = 0; q < comps; ++q) {
-        double h = 0.0, l = 0.0, a = 0.0;
-        for (int i = threadIdx.x; i < nrec; i += blockDim.x) {
-            const double* p = partial + (size_t)i * stride + 3 * q;
-            dd_add(h, l, p[0], p[1]);
-            a += p[2];
-        }
-        block_reduce_dd(h, l, a, red);
-        if (threadIdx.x == 0) {
-            out[3 * q + 0] = h;
-            out[3 * q + 1] = l;
-            out[3 * q + 2] = a;
-        }
-        __syncthreads();
-    }
+    double rec[6];
+    reduce_partials(partial, nrec, stride, comps, rec, red);
+    if (threadIdx.x == 0)
+        for (int i = 0; i < 3 * comps; ++i) out[i] = rec[i];
 }
 
 // ---------------------------------------------------------------------------

@@ -65,25 +65,6 @@ int_dense_kernel(const int* __restrict__ M,        // [2][N][N]: +2A then -2A, c
     }
 }
 
-// Sum of the per-block records mod 2^128 (one block, fixed order).
-__global__ void __launch_bounds__(256)
-reduce_i128_kernel(const unsigned long long* __restrict__ partial, int nrec, unsigned long long* __restrict__ out)
-{
-    __shared__ unsigned long long red[2 * 256];
-    unsigned __int128 t = 0;
-    for (int i = threadIdx.x; i < nrec; i += blockDim.x)
-        t += ((unsigned __int128)partial[2 * i + 1] << 64) | partial[2 * i];
-    red[2 * threadIdx.x] = (unsigned long long)t;
-    red[2 * threadIdx.x + 1] = (unsigned long long)(t >> 64);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned __int128 s = 0;
-        for (int i = 0; i < (int)blockDim.x; ++i) s += ((unsigned __int128)red[2 * i + 1] << 64) | red[2 * i];
-        out[0] = (unsigned long long)s;
-        out[1] = (unsigned long long)(s >> 64);
-    }
-}
-
 template <int N>
 const void* int_ptr()
 {
@@ -106,6 +87,5 @@ const void* int_dense_kernel_ptr(int n)
     return ints::int_lookup(n, std::make_integer_sequence<int, kMaxN>{});
 }
 
-const void* reduce_i128_kernel_ptr() { return reinterpret_cast<const void*>(&ints::reduce_i128_kernel); }
 
 }  // namespace spm

@@ -323,39 +323,6 @@ int_prune_kernel(const int* __restrict__ blob_, const unsigned long long* __rest
     }
 }
 
-// The per-block records summed mod 2^128, and the task counters set back to
-// 0 for the plan's next run (one block).
-__global__ void __launch_bounds__(256)
-reduce_prune_kernel(const unsigned long long* __restrict__ partial, int nrec, unsigned long long* __restrict__ out,
-                    unsigned int* __restrict__ counter, int counters)
-{
-    __shared__ unsigned long long red[2 * (256 / kWave)];
-    for (int i = threadIdx.x; i < counters; i += 256) counter[i * kPruneCounterStride] = 0u;
-    unsigned __int128 t = 0;
-    for (int i = threadIdx.x; i < nrec; i += 256)
-        t += ((unsigned __int128)partial[2 * i + 1] << 64) | partial[2 * i];
-    unsigned long long lo = (unsigned long long)t, hi = (unsigned long long)(t >> 64);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const unsigned long long olo = __shfl_xor(lo, off, kWave);
-        const unsigned long long ohi = __shfl_xor(hi, off, kWave);
-        const unsigned long long s = lo + olo;
-        hi = hi + ohi + (s < lo ? 1ull : 0ull);
-        lo = s;
-    }
-    if ((threadIdx.x & (kWave - 1)) == 0) {
-        red[2 * (threadIdx.x / kWave)] = lo;
-        red[2 * (threadIdx.x / kWave) + 1] = hi;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned __int128 s = 0;
-        for (int i = 0; i < 256 / kWave; ++i) s += ((unsigned __int128)red[2 * i + 1] << 64) | red[2 * i];
-        out[0] = (unsigned long long)s;
-        out[1] = (unsigned long long)(s >> 64);
-    }
-}
-
 template <int FB, int NQ>
 const void* ptr(bool nodes)
 {
@@ -384,7 +351,5 @@ const void* int_prune_kernel_ptr(int field_bytes, int dwords, bool nodes)
     default: return nullptr;
     }
 }
-
-const void* reduce_prune_kernel_ptr() { return reinterpret_cast<const void*>(&prune::reduce_prune_kernel); }
 
 }  // namespace spm

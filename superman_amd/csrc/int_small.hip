@@ -1,8 +1,7 @@
 // int_small.hip -- single-matrix exact Ryser for integer matrices with small
 // row sums (every sum_j |a_ij| < 2^B, B = bit width of n; all 0/1 matrices),
 // walked in FP64 with exact grouped products (walk_intfp.h).  Same task
-// loop, block sum mod 2^128 and per-block records as int_dense.hip, whose
-// final reduction kernel (reduce_i128_kernel) it shares.
+// loop, block sum mod 2^128 and per-block records as int_dense.hip.
 #include "walk_intfp.h"
 
 #ifndef SPM_INTFP_ONLY_N

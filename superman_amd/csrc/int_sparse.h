@@ -3,7 +3,7 @@
 // walk_sparse.h; this file holds the grid-strided task loop over one
 // matrix's chunks (each wave with its queue of deferred products in LDS),
 // the final flush of the queues and the block sum mod 2^128 into per-block
-// records, which int_dense.hip's reduce_i128_kernel sums.  The orders are
+// records, which run_io.hip's run_end_i128_kernel sums.  The orders are
 // instantiated in several translation units (int_sparse*.hip), which the
 // build compiles in parallel: each order's kernel takes 10-30 s to compile.
 #ifndef SPM_INT_SPARSE_H

@@ -23,6 +23,23 @@ int dense_f64_unroll_bits(int n);
 //   args: (const double* partial, int nrec, int stride, int comps, double* out)
 const void* reduce_partials_kernel_ptr();
 
+// run_io.hip -- the first and last kernel of a plan's run.
+struct RunResult {              // pinned host memory
+    unsigned long long word[6]; // hi, lo, abs per component, or T mod 2^128 (lo, hi)
+    unsigned long long ticks;   // device time from begin to end, 100 MHz
+    unsigned int flag;          // the run's sequence number, stored last
+    unsigned int pad;
+};
+//   begin: (const uint4* src, uint4* dst, unsigned words, uint4* zero, unsigned
+//          zwords, unsigned long long* t0), 256 threads
+//   end:   (const double* partial, int nrec, int stride, int comps, const
+//          unsigned long long* t0, RunResult* host, unsigned seq) or (const
+//          unsigned long long* partial, int nrec, t0, host, seq), one block
+//          of 256
+const void* run_begin_kernel_ptr();
+const void* run_end_dd_kernel_ptr();
+const void* run_end_i128_kernel_ptr();
+
 // dense_pair.hip -- the same arguments for a matrix whose column 0 is all
 // ones; orders kPairMinN..kMaxN, L >= kPairMinChunk.
 const void* dense_pair_kernel_ptr(int n, bool compensated);
@@ -40,8 +57,6 @@ const void* dense_c128_kernel_ptr(int n, bool compensated);
 //          unsigned long long* partial /* [grid][2] */, uint64_t task_begin,
 //          uint64_t task_end, uint64_t num_chunks, int L, int accumulate)
 const void* int_dense_kernel_ptr(int n);
-//   args: (const unsigned long long* partial, int nrec, unsigned long long* out /* [2] */)
-const void* reduce_i128_kernel_ptr();
 
 // int_small.hip -- exact walk in FP64 for integer matrices whose absolute
 // row sums are all below 2^int_small_bits(n) (every 0/1 matrix); same
@@ -83,12 +98,8 @@ constexpr int kSparseSlots = 7;  // entries per record
 //          walks the listed nodes, with out_count as its work counters.
 //          Lists have kPruneSets segments of cap prefixes; a set of counters
 //          is kPruneSets lines, all 0 before the run.
-//   reduce: (const unsigned long long* partial, int nrec, unsigned long long*
-//          out /* [2] */, unsigned int* counter, int counters), which sets
-//          the counters back to 0
 // field_bytes 1 (dwords 4, 8, 12, 16) or 2 (dwords 8, 16, 24).
 const void* int_prune_kernel_ptr(int field_bytes, int dwords, bool nodes);
-const void* reduce_prune_kernel_ptr();
 constexpr int kPruneBlock = 512;
 constexpr int kPruneLevels = 12;      // column groups of 6 of 62 walked columns, and one
 constexpr int kPruneTopBits = 15;     // the first launch has at most 2^15 prefixes
