@@ -40,6 +40,7 @@ SOURCES = [  # the longest compiles first, so that the job pool starts them earl
     ("int_sparse_57.hip", []),
     ("int_sparse_49.hip", []),
     ("int_sparse_46.hip", []),
+    ("dense_c128_pair.hip", []),
     ("dense_c128.hip", []),
     ("int_sparse_17.hip", []),
     ("batch.hip", []),

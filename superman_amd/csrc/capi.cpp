@@ -158,9 +158,9 @@ void gray_geometry(int n, int unroll_bits, int64_t resident_waves, int* L, uint6
     *tasks = (*chunks + kWaveLanes - 1) / kWaveLanes;
 }
 
-void pair_geometry(int n, int64_t resident_waves, int* L, uint64_t* chunks, uint64_t* tasks)
+void pair_geometry(int n, int64_t resident_waves, int* L, uint64_t* chunks, uint64_t* tasks, GrayWalk walk)
 {
-    gray_geometry(n, dense_f64_unroll_bits(n), resident_waves, L, chunks, tasks, GrayWalk::kReal);
+    gray_geometry(n, walk == GrayWalk::kReal ? dense_f64_unroll_bits(n) : 1, resident_waves, L, chunks, tasks, walk);
     *L = std::max(*L, kPairMinChunk);
     *chunks = uint64_t(1) << (n - 1 - *L);
     *tasks = (*chunks + kWaveLanes - 1) / kWaveLanes;
@@ -202,7 +202,7 @@ struct spm_plan {
     size_t counter_bytes = 0;            // zeroed at the start of every run
     double log2_bound = 0;   // integer kind: log2 of the bound on |T|
     int halved = 0;          // integer kinds: rows carried halved (int_row_weights)
-    bool pair = false;       // dense real plans: the matrix is scaled for dense_pair_kernel
+    bool pair = false;       // dense plans: the matrix is scaled for a pair kernel
     PairScale scale;
     int log2_scale = 0;      // FP32-product plans: perm = 2^log2_scale perm(scaled)
     double* d_partial = nullptr;
@@ -353,18 +353,23 @@ static void dense_grid(spm_plan* p)
     dense_launch_shape(p->kind, p->n, p->precision, p->tasks, p->max_grid, &p->grid, &p->slices);
 }
 
+static const void* pair_kernel_ptr(int kind, int n, bool comp)
+{
+    return kind == 1 ? dense_pair_kernel_ptr(n, comp) : dense_c128_pair_kernel_ptr(n, comp);
+}
+
 static void dense_kernel_name(spm_plan* p)
 {
-    const char* comp = p->precision == SPM_PREC_COMPENSATED ? "true" : "false";
+    const bool comp = p->precision == SPM_PREC_COMPENSATED;
     const int n = p->n, ub = dense_f64_unroll_bits(n);
+    const char* c = comp ? "true" : "false";
+    const bool pair = p->pair && p->kern == pair_kernel_ptr(p->kind, n, comp);
     char kn[96];
     if (p->precision == SPM_PREC_F32_PRODUCT) std::snprintf(kn, sizeof kn, "dense_f32p_kernel<%d, %d>", n, ub);
-    else if (p->kind == 2) std::snprintf(kn, sizeof kn, "dense_c128_kernel<%d, %s>", n, comp);
+    else if (p->kind == 2)
+        std::snprintf(kn, sizeof kn, "%s<%d, %s>", pair ? "dense_c128_pair_kernel" : "dense_c128_kernel", n, c);
     else
-        std::snprintf(kn, sizeof kn, "%s<%d, %d, %s>",
-                      p->kern == dense_pair_kernel_ptr(n, p->precision == SPM_PREC_COMPENSATED) ? "dense_pair_kernel"
-                                                                                                : "dense_f64_kernel",
-                      n, ub, comp);
+        std::snprintf(kn, sizeof kn, "%s<%d, %d, %s>", pair ? "dense_pair_kernel" : "dense_f64_kernel", n, ub, c);
     p->kname = kn;
 }
 
@@ -394,10 +399,11 @@ static int make_dense_plan(int kind, const double* a, int n, int precision, int 
     p->precision = precision;
     p->device = device;
     const bool comp = precision == SPM_PREC_COMPENSATED;
-    std::vector<double> scaled((size_t)(kind == 1 ? n * n : 0));
-    p->pair = kind == 1 && !f32p && pair_prepare(a, n, scaled.data(), &p->scale);
+    std::vector<double> scaled((size_t)w * n * n);
+    p->pair = !f32p && (kind == 1 ? pair_prepare(a, n, scaled.data(), &p->scale)
+                                  : pair_prepare_complex(a, n, scaled.data()));
     if (p->pair) a = scaled.data();
-    p->kern = p->pair ? dense_pair_kernel_ptr(n, comp) : f32p ? dense_f32p_kernel_ptr(n) : kind == 1 ? dense_f64_kernel_ptr(n, comp) : dense_c128_kernel_ptr(n, comp);
+    p->kern = p->pair ? pair_kernel_ptr(kind, n, comp) : f32p ? dense_f32p_kernel_ptr(n) : kind == 1 ? dense_f64_kernel_ptr(n, comp) : dense_c128_kernel_ptr(n, comp);
     p->rec = kind == 1 ? 4 : 8;
     p->comps = kind == 1 ? 1 : 2;
     if (!p->kern) {
@@ -412,8 +418,9 @@ static int make_dense_plan(int kind, const double* a, int n, int precision, int 
     }
     const int64_t waves = int64_t(bpc) * cus * (kDenseBlock / kWaveLanes);
     const int ub = kind == 1 ? dense_f64_unroll_bits(n) : (n >= 3 ? 1 : 0);
-    if (p->pair) pair_geometry(n, waves, &p->L, &p->chunks, &p->tasks);
-    else gray_geometry(n, ub, waves, &p->L, &p->chunks, &p->tasks, kind == 1 ? GrayWalk::kReal : GrayWalk::kComplex);
+    const GrayWalk walk = kind == 1 ? GrayWalk::kReal : GrayWalk::kComplex;
+    if (p->pair) pair_geometry(n, waves, &p->L, &p->chunks, &p->tasks, walk);
+    else gray_geometry(n, ub, waves, &p->L, &p->chunks, &p->tasks, walk);
     p->max_grid = bpc * cus;
     dense_grid(p);
     dense_kernel_name(p);
@@ -898,7 +905,7 @@ static int dense_run(spm_plan* p, hipStream_t st, spm_result* r)
 
     std::memset(r, 0, sizeof *r);
     const int n = p->n;
-    if (p->pair) pair_finish(p->scale, rec);
+    if (p->pair && p->kind == 1) pair_finish(p->scale, rec);
     dense_fill_result(n, p->comps == 2, p->precision != SPM_PREC_PLAIN, rec, r);
     if (p->precision == SPM_PREC_F32_PRODUCT) f32prod_finish(n, p->log2_scale, r);
     r->status = SPM_OK;
@@ -1015,7 +1022,8 @@ extern "C" int spm_plan_set_log2_chunk(spm_plan* p, int L)
     if (L < lo || L > B) return SPM_EINVAL;
     if (p->pair) {  // the scaled matrix by either kernel: shorter chunks one subset at a time
         const bool comp = p->precision == SPM_PREC_COMPENSATED;
-        p->kern = L >= kPairMinChunk ? dense_pair_kernel_ptr(n, comp) : dense_f64_kernel_ptr(n, comp);
+        p->kern = L >= kPairMinChunk ? pair_kernel_ptr(p->kind, n, comp)
+                  : p->kind == 1 ? dense_f64_kernel_ptr(n, comp) : dense_c128_kernel_ptr(n, comp);
         dense_kernel_name(p);
     }
     p->L = L;

@@ -39,15 +39,18 @@ namespace {
 
 // Whether sums of a row's entries are exact in FP64 (entries of few bits, such
 // as integers): then x has no rounding to lose.
-bool exact_sums(const double* a, int n)
+bool exact_sums(const double* a, int entries)
 {
-    int top = -5000, low = 5000;
-    for (int e = 0; e < n * n; ++e) {
-        if (a[e] == 0.0) continue;
-        int x;
-        const int64_t m = (int64_t)std::ldexp(std::frexp(a[e], &x), 53);
-        top = std::max(top, x);
-        low = std::min(low, x - 53 + __builtin_ctzll((unsigned long long)m));
+    int top = -1, low = 1 << 20;  // in bits above 2^-1074
+    for (int e = 0; e < entries; ++e) {
+        uint64_t u;
+        std::memcpy(&u, a + e, 8);
+        const int x = (int)((u >> 52) & 0x7ff);
+        const uint64_t m = (u & ((uint64_t(1) << 52) - 1)) | (x ? uint64_t(1) << 52 : 0);
+        if (m == 0) continue;
+        const int unit = std::max(x, 1) - 1;
+        top = std::max(top, unit + 53);
+        low = std::min(low, unit + __builtin_ctzll(m));
     }
     return top + 7 - low <= 53;  // 2 n entries and a half
 }
@@ -56,6 +59,20 @@ bool power_of_two(double v)
 {
     int x;
     return std::fabs(std::frexp(v, &x)) == 0.5;
+}
+
+// The allowed column with the largest `least`, if that is above 2^-60.
+template <class Allowed>
+int pivot_column(const double* least, int n, Allowed allowed)
+{
+    int col = -1;
+    double best = 0x1p-60;
+    for (int j = 0; j < n; ++j)
+        if (least[j] > best && allowed(j)) {
+            best = least[j];
+            col = j;
+        }
+    return col;
 }
 
 }  // namespace
@@ -74,28 +91,21 @@ bool power_of_two(double v)
 bool pair_prepare(const double* a, int n, double* out, PairScale* scale)
 {
     if (n < kPairMinN) return false;
-    const bool exact = exact_sums(a, n);
-    double rowmax[kMaxN];
+    const bool exact = exact_sums(a, n * n);
+    double least[kMaxN];  // per column: the smallest |a_ij| / max_k |a_ik|
+    std::fill(least, least + n, 1.0);
     for (int i = 0; i < n; ++i) {
-        rowmax[i] = 0.0;
-        for (int j = 0; j < n; ++j) rowmax[i] = std::max(rowmax[i], std::fabs(a[(size_t)i * n + j]));
-        if (rowmax[i] == 0.0) return false;
+        const double* r = a + (size_t)i * n;
+        double top = 0.0;
+        for (int j = 0; j < n; ++j) top = std::max(top, std::fabs(r[j]));
+        if (top == 0.0) return false;
+        for (int j = 0; j < n; ++j) least[j] = std::min(least[j], std::fabs(r[j]) / top);
     }
-    int col = -1;
-    double best = 0x1p-60;
-    for (int j = 0; j < n; ++j) {
-        double least = 1.0;
-        bool two = true;
-        for (int i = 0; i < n && least > best; ++i) {
-            const double v = a[(size_t)i * n + j];
-            least = std::min(least, std::fabs(v) / rowmax[i]);
-            two = two && (!exact || power_of_two(v));
-        }
-        if (least > best && two) {
-            best = least;
-            col = j;
-        }
-    }
+    const int col = pivot_column(least, n, [&](int j) {
+        for (int i = 0; exact && i < n; ++i)
+            if (!power_of_two(a[(size_t)i * n + j])) return false;
+        return true;
+    });
     if (col < 0) return false;
     double bound = 0.0, sh = 1.0, sl = 0.0;
     int exp2 = 0;
@@ -126,6 +136,75 @@ bool pair_prepare(const double* a, int n, double* out, PairScale* scale)
     scale->lo = sl;
     scale->exp2 = exp2;
     return true;
+}
+
+// The complex matrix (interleaved re, im) for dense_c128_pair_kernel: rows 0
+// to n-3 divided by their entry c_i of one column, which comes first, row n-2
+// times the product of those c_i, the last row as it is.  The product of a
+// term's rows, of its first n-1 rows and its last row are then those of `a`,
+// so the sums, |term| bounds included, need no scaling.  Entries are rounded
+// once, from long double: with the factors rounded to double first (2 us less
+// at order 21) Haar orders 12 and 16 lost 1.2x against 64 bits.  The column
+// and the cases it is refused for are pair_prepare's; an exact matrix needs a
+// column of +-2^k, +-i 2^k.
+bool pair_prepare_complex(const double* a, int n, double* out)
+{
+    if (n < kPairMinN) return false;
+    const bool exact = exact_sums(a, 2 * n * n);
+    double least[kMaxComplexN];
+    std::fill(least, least + n, 1.0);
+    for (int i = 0; i < n; ++i) {
+        const double* r = a + (size_t)2 * n * i;
+        double top = 0.0;
+        for (int e = 0; e < 2 * n; ++e) top = std::max(top, std::fabs(r[e]));
+        if (top == 0.0) return false;
+        for (int j = 0; i + 2 < n && j < n; ++j)
+            least[j] = std::min(least[j], std::max(std::fabs(r[2 * j]), std::fabs(r[2 * j + 1])) / top);
+    }
+    const int col = pivot_column(least, n, [&](int j) {
+        for (int i = 0; exact && i + 2 < n; ++i) {
+            const double re = a[(size_t)2 * (i * n + j)], im = a[(size_t)2 * (i * n + j) + 1];
+            if (!(re == 0.0 ? power_of_two(im) : im == 0.0 && power_of_two(re))) return false;
+        }
+        return true;
+    });
+    if (col < 0) return false;
+    double bound = 0.0;
+    long double kr = 1.0L, ki = 0.0L;  // the product of the c_i
+    for (int i = 0; i < n; ++i) {
+        const double* r = a + (size_t)2 * n * i;
+        long double fr = 1.0L, fi = 0.0L;  // the row's factor
+        if (i + 2 < n) {
+            const long double cr = r[2 * col], ci = r[2 * col + 1], d = cr * cr + ci * ci;
+            fr = cr / d;
+            fi = -ci / d;
+            const long double t = kr * cr - ki * ci;
+            ki = kr * ci + ki * cr;
+            kr = t;
+        } else if (i + 2 == n) {
+            const long double m = std::fabs(kr) + std::fabs(ki);
+            if (!(m >= 0x1p-450L && m <= 0x1p450L)) return false;
+            fr = kr;
+            fi = ki;
+        }
+        double sum = 0.0;
+        double* o = out + (size_t)2 * n * i;
+        for (int j = 0; j < n; ++j) {
+            const double re = r[2 * j], im = r[2 * j + 1];
+            o[2 * j] = i + 1 < n ? (double)(re * fr - im * fi) : re;
+            o[2 * j + 1] = i + 1 < n ? (double)(re * fi + im * fr) : im;
+            sum += std::fabs(o[2 * j]) + std::fabs(o[2 * j + 1]);
+        }
+        std::swap(o[0], o[2 * col]);
+        std::swap(o[1], o[2 * col + 1]);
+        if (i + 2 < n) {
+            o[0] = 1.0;
+            o[1] = 0.0;
+        }
+        if (i + 2 < n) bound += std::log2(sum);
+        if (!(sum <= 0x1p500)) return false;
+    }
+    return bound <= 450.0;
 }
 
 // rec = (hi, lo, abs) times the scale.

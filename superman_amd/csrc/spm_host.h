@@ -25,8 +25,9 @@ double now_seconds();
 enum class GrayWalk { kOther, kReal, kComplex };
 void gray_geometry(int n, int unroll_bits, int64_t resident_waves, int* L, uint64_t* chunks, uint64_t* tasks,
                    GrayWalk walk = GrayWalk::kOther);
-// The same for dense_pair_kernel, whose chunks are at least 2^kPairMinChunk.
-void pair_geometry(int n, int64_t resident_waves, int* L, uint64_t* chunks, uint64_t* tasks);
+// The same for the pair kernels, whose chunks are at least 2^kPairMinChunk.
+void pair_geometry(int n, int64_t resident_waves, int* L, uint64_t* chunks, uint64_t* tasks,
+                   GrayWalk walk = GrayWalk::kReal);
 // Grid and launch slices of a dense walk over `tasks` wave tasks (kind 1
 // real, 2 complex, 5 generated real): as many blocks as the tasks fill, at
 // most max_grid (the resident ones); runs longer than ~4 s of VALU work are
@@ -72,6 +73,8 @@ struct PairScale {
 };
 bool pair_prepare(const double* a, int n, double* scaled, PairScale* scale);
 void pair_finish(const PairScale& scale, double* rec);
+// The same for dense_c128_pair_kernel; perm(a) = perm(scaled).
+bool pair_prepare_complex(const double* a, int n, double* scaled);
 // w: per-row weights from int_row_weights (1 = row carried halved, 2 =
 // not); nullptr = every row 2 (the batch engine's layout).
 int int_row_weights(const int64_t* a, int n, unsigned char* w);

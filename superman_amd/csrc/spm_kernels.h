@@ -51,6 +51,9 @@ constexpr int kPairMinChunk = 3;
 // partial record is 8 doubles (re hi, lo, abs, im hi, lo, 0, 0, 0).
 constexpr int kMaxComplexN = 63;
 const void* dense_c128_kernel_ptr(int n, bool compensated);
+// dense_c128_pair.hip -- for matrices of pair_prepare_complex; orders
+// kPairMinN.., L >= kPairMinChunk.
+const void* dense_c128_pair_kernel_ptr(int n, bool compensated);
 
 // int_dense.hip -- exact integer walk.
 //   args: (const int* M /* [2][n][n]: +2A, -2A column-major */, const int* y0,

@@ -215,15 +215,74 @@ __device__ __forceinline__ void add_term(const double (&x)[2 * N], bool negative
     finish_term<N, COMP>(x, p, negative, br, bi, babs);
 }
 
+// Two subsets per step, for a matrix whose column 0 is (1, 0) in rows
+// 0..N-3 (pair_prepare_complex): x gives the terms of the subset without
+// column 0 and of the one with it, prod_r x_r and prod_r (x_r + a_r0), so the
+// walk never adds column 0.  p <- p x_r is a complex product; q <- q (x_r + 1) =
+// q x_r + q is one too, four FMAs; rows N-2 and N-1 add their entry z of
+// column 0 first.  Two chains each: four products in flight, in the registers
+// of the four chains of Prod.
+struct PairProd {
+    double pr[2], pi[2], qr[2], qi[2];
+};
+
+template <int N, int R0, int R1>
+__device__ __forceinline__ void prod_rows(const double (&x)[2 * N], PairProd& p, const double (&z)[4])
+{
+    static_for<R0, (R1 < N - 1 ? R1 : N - 1)>([&](auto RR) __attribute__((always_inline)) {
+        constexpr int r = decltype(RR)::value, k = r & 1;
+        const double xr = x[2 * r], xi = x[2 * r + 1];
+        if constexpr (r < 2) {
+            p.pr[k] = xr;
+            p.pi[k] = xi;
+            p.qr[k] = xr + 1.0;
+            p.qi[k] = xi;
+        } else {
+            cmul(p.pr[k], p.pi[k], xr, xi);
+            if constexpr (r == N - 2) {
+                cmul(p.qr[k], p.qi[k], xr + z[0], xi + z[1]);
+            } else {
+                const double u = __builtin_fma(p.qr[k], xr, p.qr[k]), v = __builtin_fma(p.qr[k], xi, p.qi[k]);
+                p.qr[k] = __builtin_fma(-p.qi[k], xi, u);
+                p.qi[k] = __builtin_fma(p.qi[k], xr, v);
+            }
+        }
+    });
+}
+
+// blk += sign * (P x[N-1] - Q (x[N-1] + z)), each term's modulus bounded as
+// finish_term does.
+template <int N, bool COMP>
+__device__ __forceinline__ void finish_pair(const double (&x)[2 * N], PairProd& p, const double (&z)[4], bool negative,
+                                            double& br, double& bi, double& babs)
+{
+    cmul(p.pr[0], p.pi[0], p.pr[1], p.pi[1]);
+    cmul(p.qr[0], p.qi[0], p.qr[1], p.qi[1]);
+    auto term = [&](double pr, double pi, double lr, double li, bool neg) __attribute__((always_inline)) {
+        const double sr = neg ? -pr : pr, si = neg ? -pi : pi;
+        br = __builtin_fma(sr, lr, br);
+        br = __builtin_fma(-si, li, br);
+        bi = __builtin_fma(sr, li, bi);
+        bi = __builtin_fma(si, lr, bi);
+        if constexpr (COMP) {
+            const double pa = __builtin_fabs(pr) + __builtin_fabs(pi);
+            const double la = __builtin_fabs(lr) + __builtin_fabs(li);
+            babs = __builtin_fma(pa, la, babs);
+        }
+    };
+    term(p.pr[0], p.pi[0], x[2 * N - 2], x[2 * N - 1], negative);
+    term(p.qr[0], p.qi[0], x[2 * N - 2] + z[2], x[2 * N - 1] + z[3], !negative);
+}
+
 // One Gray step: x += column `col` (x = fma(s, column, x) when FMA: the
 // per-lane direction of the special flip), whose part 0 is in `buf`, then
 // the term of the new subset.  Leaves part 0 of `next` loading into `buf`.
-template <int N, bool COMP, bool FMA>
+template <int N, bool COMP, bool FMA, bool PAIR>
 __device__ __forceinline__ void gray_step(double (&x)[2 * N], Part<N>& buf, const double* col, double s,
-                                          const double* next, bool negative, double& br, double& bi,
-                                          double& babs)
+                                          const double* next, bool negative, const double (&z)[4], double& br,
+                                          double& bi, double& babs)
 {
-    Prod p;
+    std::conditional_t<PAIR, PairProd, Prod> p;
     static_for<0, kPhases<N>>([&](auto PP) __attribute__((always_inline)) {
         constexpr int ph = decltype(PP)::value;
         constexpr int r0 = ph * kPhaseRows<N>;
@@ -237,28 +296,42 @@ __device__ __forceinline__ void gray_step(double (&x)[2 * N], Part<N>& buf, cons
         if constexpr (ph + 1 < kPhases<N>) load_part<N, ph + 1>(buf, col);
         else load_part<N, 0>(buf, next);
         fence();
-        prod_rows<N, r0, r1>(x, p);
-        if constexpr (ph + 1 == kPhases<N>) finish_term<N, COMP>(x, p, negative, br, bi, babs);
+        if constexpr (PAIR) {
+            prod_rows<N, r0, r1>(x, p, z);
+            if constexpr (ph + 1 == kPhases<N>) finish_pair<N, COMP>(x, p, z, negative, br, bi, babs);
+        } else {
+            prod_rows<N, r0, r1>(x, p);
+            if constexpr (ph + 1 == kPhases<N>) finish_term<N, COMP>(x, p, negative, br, bi, babs);
+        }
         fence();
     });
 }
 
 // One lane's chunk: the 2^L Gray steps starting at k = h 2^L, folded into the
 // caller's compensated sums (re_hi + re_lo, im_hi + im_lo; abs_sum bounds
-// sum |term| in the L1 norm, COMP only).
-template <int N, bool COMP>
+// sum |term| in the L1 norm, COMP only).  PAIR: a chunk of 2^L steps of two
+// subsets each over columns 1..N-2, L >= 2.
+template <int N, bool COMP, bool PAIR = false>
 __device__ __forceinline__ void walk_c128(const double* __restrict__ M,   // [2][N][2N]: +A, -A
                                           const double* __restrict__ x0,  // 2N doubles
                                           uint64_t h, int L, double& re_hi, double& re_lo, double& im_hi,
                                           double& im_lo, double& abs_sum)
 {
     constexpr int C = 2 * N;  // doubles per column
+    constexpr int NC = PAIR ? N - 2 : N - 1;  // walked columns
+    double z[4] = {0.0, 0.0, 0.0, 0.0};
+    if constexpr (PAIR) {
+        const const_f64* __restrict__ c0 = step_ptr(M) + 2 * (N - 2);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z[i] = c0[i];
+        M += C;
+    }
     const double* Mneg = M + (size_t)N * C;
     double x[C];
     stream_column<N, 0>(x, x0, 0.0);
     const uint64_t k0 = h << L;
     const uint64_t g0 = k0 ^ (k0 >> 1);
-    for (int j = (L > 0 ? L - 1 : 0); j < N - 1; ++j) {
+    for (int j = (L > 0 ? L - 1 : 0); j < NC; ++j) {
         const double b = ((g0 >> j) & 1u) ? 1.0 : 0.0;
         stream_column<N, 2>(x, M + (size_t)j * C, b);
     }
@@ -283,7 +356,7 @@ __device__ __forceinline__ void walk_c128(const double* __restrict__ M,   // [2]
         add_term<N, COMP>(x, false, br, bi, babs);
         Part<N> buf;
         load_part<N, 0>(buf, M);
-        gray_step<N, COMP, true>(x, buf, M, lane_sign, M, true, br, bi, babs);
+        gray_step<N, COMP, true, false>(x, buf, M, lane_sign, M, true, z, br, bi, babs);
     } else {
         // 2-step blocks as in dense_f64 (L >= 2): k = 2m flips column
         // ctz(m)+1, k = 2m+1 flips column 0; block nblk/2 (column L-1)
@@ -295,18 +368,24 @@ __device__ __forceinline__ void walk_c128(const double* __restrict__ M,   // [2]
             return (((m >> (tz + 1)) & 1u) ? Mneg : M) + (size_t)(tz + 1) * C;
         };
         Part<N> buf;
-        add_term<N, COMP>(x, false, br, bi, babs);  // k = 0
+        if constexpr (PAIR) {  // k = 0
+            PairProd p;
+            prod_rows<N, 0, N>(x, p, z);
+            finish_pair<N, COMP>(x, p, z, false, br, bi, babs);
+        } else {
+            add_term<N, COMP>(x, false, br, bi, babs);
+        }
         load_part<N, 0>(buf, M);
         const double* pa = a_col(1);
         fence();
-        gray_step<N, COMP, false>(x, buf, M, 1.0, pa, true, br, bi, babs);  // k = 1: +column 0
+        gray_step<N, COMP, false, PAIR>(x, buf, M, 1.0, pa, true, z, br, bi, babs);  // k = 1: +column 0
         auto block = [&](uint32_t m, auto SPECIAL) __attribute__((always_inline)) {
             const double* pb = (m & 1u) ? Mneg : M;
-            gray_step<N, COMP, decltype(SPECIAL)::value>(x, buf, pa, lane_sign, pb, false, br, bi, babs);
-            pa = a_col(m + 1);  // m+1 = nblk: column L <= N-1, a valid address
-            gray_step<N, COMP, false>(x, buf, pb, 1.0, pa, true, br, bi, babs);
+            gray_step<N, COMP, decltype(SPECIAL)::value, PAIR>(x, buf, pa, lane_sign, pb, false, z, br, bi, babs);
+            pa = a_col(m + 1);  // m+1 = nblk: column L <= NC, a valid address
+            gray_step<N, COMP, false, PAIR>(x, buf, pb, 1.0, pa, true, z, br, bi, babs);
         };
-        constexpr uint32_t G = kFoldSteps / 2;
+        constexpr uint32_t G = (PAIR ? kFoldSteps / 2 : kFoldSteps) / 2;
         auto run = [&](uint32_t m, uint32_t end) __attribute__((always_inline)) {
             while (m < end) {
                 const uint32_t mend = min(end, (m | (G - 1)) + 1);
