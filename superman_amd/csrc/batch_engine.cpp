@@ -137,18 +137,45 @@ namespace {
 
 bool dry(const spm_batch* b) { return b->cfg.executor == SPM_EXEC_DRYRUN; }
 
+// The default tuning.  One fused launch: every request's items are in the
+// work queue at once, where the three one-kind kernels run one after another
+// and each ends in its own thinly filled tail (256 mixed requests of orders 8
+// to 24: 2.45 -> 2.08 ms, 64 of orders 8 to 20: 0.94 -> 0.51 ms, 24 of orders
+// 4 to 14: 0.32 -> 0.18 ms).  Chunks of 2^8 complex and 2^9 integer steps: the
+// last item to start ends a batch, and with 2^9 and 2^10 steps 48 requests of
+// orders 10 to 25 took 1.04 instead of 0.95 ms; chunks half as long again (and
+// 2^8 real ones) spend more on chunk starts (400 requests 4.1 -> 4.4 ms).
+constexpr int kBatchFused = 1;
+constexpr int kBatchChunk[4] = {0, 10, 8, 9};  // [kind]
+// Chunk sizes of a request whose items at those sizes exceed the engine's.
+constexpr int kBatchChunkWide[4] = {0, 10, 9, 10};
+// A request is split over up to 2^10 chunks (16 wavefronts) before its chunks
+// grow beyond 2^5 steps, since one wavefront's serial walk bounds a batch of
+// small orders: 32 requests of orders 4 to 16 take 0.21 instead of 0.26 ms.  2^12 chunks cost
+// 400 requests of orders 8 to 25 2 % (4.13 -> 4.20 ms) in chunk starts.
+constexpr int kSplitChunks = 10;
+constexpr int kSplitSteps = 5;
+
 // Chunk size for a request: L >= 2 for the pipelined walks (n >= 3); n = 2
-// walks one 2-step chunk per lane (L = 1) and n = 1 its single subset.
+// walks one 2-step chunk per lane (L = 1) and n = 1 its single subset.  It
+// follows from the request and the engine's configuration alone.
 void geometry(const spm_batch* b, Req* r)
 {
     const int B = r->n - 1;
+    const int target = b->tune.log2_chunk[r->kind];
+    auto items = [&](int L) { return ((uint64_t(1) << (B - L)) + kWaveLanes - 1) / kWaveLanes; };
     int L;
     if (r->n == 1) L = 0;
     else if (r->n == 2) L = 1;
-    else L = std::max(2, std::min({b->tune.log2_chunk[r->kind], B - 6, B}));
+    else {
+        const int whole = std::max(2, std::min(target, B - 6));  // at least one full wavefront
+        L = std::min(whole, std::max(kSplitSteps, B - kSplitChunks));
+        if (items(L) > (uint64_t)b->cfg.max_items)
+            L = target == kBatchChunk[r->kind] ? std::max(2, std::min(kBatchChunkWide[r->kind], B - 6)) : whole;
+    }
     r->L = L;
     r->chunks = uint64_t(1) << (B - L);
-    r->items = (uint32_t)((r->chunks + kWaveLanes - 1) / kWaveLanes);
+    r->items = (uint32_t)items(L);
     const double ops = ops_per_subset(r->dev_kind, r->n);
     r->work = std::ldexp(1.0, B) * ops;
 }
@@ -730,12 +757,9 @@ extern "C" int spm_batch_create(const spm_batch_config* cfg, spm_batch** out)
     if (cfg->executor != SPM_EXEC_DEVICE && cfg->executor != SPM_EXEC_DRYRUN) return SPM_EINVAL;
     std::unique_ptr<spm_batch> b(new spm_batch);
     b->cfg = *cfg;
-    b->tune.fused = 0;
+    b->tune.fused = kBatchFused;
     b->tune.waves_per_cu = 0;
-    b->tune.log2_chunk[0] = 0;
-    b->tune.log2_chunk[SPM_KIND_REAL] = 10;
-    b->tune.log2_chunk[SPM_KIND_COMPLEX] = 9;
-    b->tune.log2_chunk[SPM_KIND_INT] = 10;
+    std::copy(kBatchChunk, kBatchChunk + 4, b->tune.log2_chunk);
     b->desc_off = align_up(sizeof(BatchHeader), kBatchAlign);
     b->item_off = align_up(b->desc_off + sizeof(BatchRequestDesc) * cfg->max_requests, kBatchAlign);
     b->data_off = align_up(b->item_off + sizeof(uint32_t) * cfg->max_items, kBatchAlign);
