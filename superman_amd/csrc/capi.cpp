@@ -212,7 +212,8 @@ struct spm_plan {
     unsigned int* d_counter = nullptr;  // its counters, a set per launch
     unsigned long long* d_list[2] = {nullptr, nullptr};
     unsigned int list_cap = 0;          // prefixes per list segment
-    int first_group = 0;                // PrunePlan::first_group
+    int first_group = 0, field_bytes = 0, dwords = 0;  // as in PrunePlan
+    char* d_table = nullptr;            // lds_bytes, as the blocks keep them in LDS
     const void* kern2 = nullptr;        // the walk over the listed nodes
     int grid2 = 0;
     std::string kname;
@@ -231,7 +232,7 @@ static void plan_free(spm_plan* p)
 
 // A plan's workspace, split into its arrays (256-byte aligned).
 static int plan_memory(spm_plan* p, size_t m_bytes, size_t x0_bytes, size_t partial_bytes, size_t counter_bytes = 0,
-                       size_t list_bytes = 0)
+                       size_t list_bytes = 0, size_t table_bytes = 0)
 {
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
     p->in_bytes = up(m_bytes) + up(x0_bytes);
@@ -245,6 +246,8 @@ static int plan_memory(spm_plan* p, size_t m_bytes, size_t x0_bytes, size_t part
     off += 256;
     const size_t list = off;
     off += 2 * up(list_bytes);
+    const size_t table = off;
+    off += up(table_bytes);
     const int rc = workspace_get(p->device, off, p->in_bytes, &p->ws);
     if (rc != SPM_OK) return rc;
     char* d = p->ws->dev;
@@ -259,6 +262,7 @@ static int plan_memory(spm_plan* p, size_t m_bytes, size_t x0_bytes, size_t part
         p->d_list[0] = (unsigned long long*)(d + list);
         p->d_list[1] = (unsigned long long*)(d + list + up(list_bytes));
     }
+    if (table_bytes) p->d_table = d + table;
     p->uploaded = p->in_bytes == 0;
     return SPM_OK;
 }
@@ -473,6 +477,8 @@ static int make_prune_plan(const PrunePlan& pr, int n, double log2_bound, int ha
     p->lds_bytes = pr.lds_bytes;
     p->tasks = pr.prefixes;
     p->first_group = pr.first_group;
+    p->field_bytes = pr.field_bytes;
+    p->dwords = pr.dwords;
     p->kern = int_prune_kernel_ptr(pr.field_bytes, pr.dwords, false);
     p->kern2 = int_prune_kernel_ptr(pr.field_bytes, pr.dwords, true);
     int bpc = 0, bpc2 = 0;
@@ -501,7 +507,7 @@ static int make_prune_plan(const PrunePlan& pr, int n, double log2_bound, int ha
     p->records = p->grid * (p->first_group - 2) + p->grid2;  // a record per block and launch
     if (plan_memory(p, sizeof(int) * pr.blob.size(), 0, sizeof(unsigned long long) * 2 * p->records,
                     sizeof(unsigned int) * kPruneSets * kPruneCounterStride * p->first_group,
-                    sizeof(unsigned long long) * p->list_cap * kPruneSets) != SPM_OK) {
+                    sizeof(unsigned long long) * p->list_cap * kPruneSets, p->lds_bytes) != SPM_OK) {
         plan_free(p);
         return SPM_ENOMEM;
     }
@@ -918,16 +924,22 @@ static int dense_run(spm_plan* p, hipStream_t st, spm_result* r)
 }
 
 // The launches of a pruned plan over the first launch's prefixes [tb, te):
-// one per column group from first_group - 1 down to 2, then the nodes.
+// the tables, one per column group from first_group - 1 down to 2, then the nodes.
 static int prune_launch(spm_plan* p, uint64_t tb, uint64_t te, hipStream_t st)
 {
     unsigned long long* list = nullptr;
     unsigned int* count = nullptr;
     unsigned long long* partial = (unsigned long long*)p->d_partial;
+    {
+        void* args[] = {&p->d_M, &p->field_bytes, &p->dwords, &p->d_table};
+        const unsigned int blocks = (unsigned int)(p->lds_bytes / 4 + 255) / 256;
+        if (hipLaunchKernel(prune_tables_kernel_ptr(), dim3(blocks), dim3(256), args, 0, st) != hipSuccess)
+            return SPM_EHIP;
+    }
     for (int group = p->first_group - 1; group >= 1; --group) {
         unsigned long long* out = p->d_list[group & 1];
         unsigned int* out_count = p->d_counter + (size_t)kPruneSets * kPruneCounterStride * (group - 1);
-        void* args[] = {&p->d_M, &list, &count, &out, &out_count, &p->list_cap, &group, &partial, &tb, &te};
+        void* args[] = {&p->d_M, &p->d_table, &list, &count, &out, &out_count, &p->list_cap, &group, &partial, &tb, &te};
         const int grid = group == 1 ? p->grid2 : p->grid;
         if (hipLaunchKernel(group == 1 ? p->kern2 : p->kern, dim3(grid), dim3(p->block), args, p->lds_bytes, st) !=
             hipSuccess)

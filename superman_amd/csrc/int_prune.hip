@@ -4,12 +4,62 @@
 //
 // What bounds it: VALU issue on the surviving nodes (about 5 instructions
 // per testable row and node of 4096 subsets) and terms (about 250
-// instructions per 64 terms at order 40); no memory but the tables each
-// block builds in LDS from a few KB.
+// instructions per 64 terms at order 40); no memory but the tables (10 to 60
+// KB, once per block).
 #include "walk_prune.h"
 
 namespace spm {
 namespace prune {
+
+// The tables that every block of the walk keeps in LDS, once in memory: built
+// by each block itself (200 instructions an entry of a zero mask, the columns'
+// fields from memory one after another) they took 13 to 18 us of every launch.
+//   group g, setting s -> packed sum of its columns' fields;
+//   row r (field r of the packed vector), sum c over the columns outside
+//   group 0 -> the settings s of group 0 whose sum with c is the row's zero.
+// One thread per dword of the first and per mask of the second.
+__global__ void __launch_bounds__(256)
+prune_tables_kernel(const int* __restrict__ blob, int field_bytes, int dwords, uint32_t* __restrict__ tables)
+{
+    const uint32_t F = 4 / (uint32_t)field_bytes, NQ = (uint32_t)dwords;
+    const uint32_t sums = (uint32_t)blob[kPruneGroups] * 64 * NQ;
+    const int B = blob[kPruneBits];
+    const int* on = blob + prune_on_at(dwords, dwords * (int)F);
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+    if (t < sums) {
+        const uint32_t q = t % NQ, s = (t / NQ) & 63u, g = t / (64 * NQ);
+        uint32_t v = 0;
+#pragma unroll
+        for (int b = 0; b < 6; ++b) {
+            const int j = 6 * (int)g + b;
+            if (j < B) v += (uint32_t)on[(2 * j + (((s >> b) & 1u) ? 0 : 1)) * dwords + (int)q];
+        }
+        tables[t] = v;
+        return;
+    }
+    const uint32_t e = t - sums, stride = (uint32_t)blob[kPruneStride];
+    if (e >= (uint32_t)blob[kPruneLeaf] * stride) return;
+    const uint32_t r = e / stride, c = e % stride;
+    const uint32_t sh = 8 * (uint32_t)field_bytes * (r % F), fm = field_bytes == 1 ? 0xffu : 0xffffu;
+    auto field = [&](uint32_t x) __attribute__((always_inline)) { return (x >> sh) & fm; };
+    uint32_t y = 0, d[6];  // the row's sum over group 0, first of the empty setting
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+        const int* col = on + 2 * b * dwords + (int)(r / F);
+        const uint32_t off = field((uint32_t)col[dwords]);
+        d[b] = field((uint32_t)col[0]) - off;
+        y += off;
+    }
+    const uint32_t zero = field((uint32_t)blob[kPruneZero + r / F]) - c;
+    unsigned long long m = y == zero ? 1ull : 0ull;
+#pragma unroll
+    for (uint32_t k = 1; k < 64; ++k) {  // in Gray order
+        const uint32_t s = k ^ (k >> 1), b = (uint32_t)__builtin_ctz(k);
+        y += ((s >> b) & 1u) ? d[b] : 0u - d[b];
+        m |= y == zero ? 1ull << s : 0ull;
+    }
+    ((unsigned long long*)(tables + sums))[e] = r < (uint32_t)blob[kPruneTested] ? m : 0ull;
+}
 
 // The tree is walked breadth first, one launch per column group from the
 // outermost, through lists of the prefixes that survive (NODES false: a wave
@@ -24,7 +74,8 @@ namespace prune {
 // `group` + 1 (group 1: the nodes) outward, [begin, end), a power of two.
 template <int FB, int NQ, bool NODES>
 __global__ void __launch_bounds__(kPruneBlock) __attribute__((amdgpu_waves_per_eu(4)))
-int_prune_kernel(const int* __restrict__ blob_, const unsigned long long* __restrict__ in,
+int_prune_kernel(const int* __restrict__ blob_, const uint4* __restrict__ tables,
+                 const unsigned long long* __restrict__ in,
                  const unsigned int* __restrict__ in_count, unsigned long long* __restrict__ out,
                  unsigned int* __restrict__ out_count, unsigned int cap, int group,
                  unsigned long long* __restrict__ partial, uint64_t begin, uint64_t end)
@@ -39,38 +90,15 @@ int_prune_kernel(const int* __restrict__ blob_, const unsigned long long* __rest
     const const_i32* blob = (const const_i32*)blob_;
     const int G = blob[kPruneGroups];
     const int nleaf = blob[kPruneLeaf], stride = blob[kPruneStride], mode = blob[kPruneMode];
-    const int B = blob[kPruneBits];
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t w = uni(threadIdx.x / kWave);
 
-    // Tables: group g, setting s -> packed sum of its columns' fields.
     uint32_t* tab = lds;
     unsigned long long* zt = (unsigned long long*)(lds + (size_t)G * 64 * NQ);
     {
-        const int* on = blob_ + prune_on_at(NQ, NQ * F);
-        for (uint32_t e = threadIdx.x; e < (uint32_t)G * 64 * NQ; e += kPruneBlock) {
-            const uint32_t q = e % NQ, s = (e / NQ) & 63u, g = e / (64 * NQ);
-            uint32_t v = 0;
-            for (int b = 0; b < 6; ++b) {
-                const int j = 6 * (int)g + b;
-                if (j < B) v += (uint32_t)on[(2 * j + (((s >> b) & 1u) ? 0 : 1)) * NQ + q];
-            }
-            tab[e] = v;
-        }
-        __syncthreads();
-        // Zero masks: row r (field r of the packed vector), sum c over the
-        // columns outside group 0 -> settings s of group 0 with c + tab = zero.
-        const int tested = blob[kPruneTested];
-        for (int r = 0; r < nleaf; ++r) {
-            const uint32_t sh = 8 * FB * (r % F), fm = FB == 1 ? 0xffu : 0xffffu;
-            const uint32_t zero = ((uint32_t)blob[kPruneZero + r / F] >> sh) & fm;
-            for (uint32_t c = (threadIdx.x + 64 * r) % kPruneBlock; c < (uint32_t)stride; c += kPruneBlock) {
-                unsigned long long m = 0;
-                for (uint32_t s = 0; s < 64; ++s)
-                    if (((tab[s * NQ + r / F] >> sh) & fm) == zero - c) m |= 1ull << s;
-                zt[r * stride + c] = r < tested ? m : 0ull;
-            }
-        }
+        const uint32_t words = ((uint32_t)G * 64 * NQ * 4 + (uint32_t)(nleaf * stride) * 8) / 16;
+#pragma unroll 4
+        for (uint32_t i = threadIdx.x; i < words; i += kPruneBlock) ((uint4*)lds)[i] = tables[i];
         __syncthreads();
     }
 
@@ -331,6 +359,8 @@ const void* ptr(bool nodes)
 }
 
 }  // namespace prune
+
+const void* prune_tables_kernel_ptr() { return reinterpret_cast<const void*>(&prune::prune_tables_kernel); }
 
 const void* int_prune_kernel_ptr(int field_bytes, int dwords, bool nodes)
 {

@@ -88,8 +88,8 @@ constexpr int kSparseSlots = 7;  // entries per record
 
 // int_prune.hip -- exact sum over the subsets with no zero row
 // (walk_prune.h).
-//   args: (const int* blob, const unsigned long long* in, const unsigned int*
-//          in_count, unsigned long long* out, unsigned int* out_count,
+//   args: (const int* blob, const uint4* tables, const unsigned long long* in,
+//          const unsigned int* in_count, unsigned long long* out, unsigned int* out_count,
 //          unsigned int cap, int group, unsigned long long* partial
 //          /* [grid][2], its own for each launch */, uint64_t begin, uint64_t
 //          end), kPruneBlock threads, dynamic LDS PrunePlan::lds_bytes, a
@@ -103,6 +103,9 @@ constexpr int kSparseSlots = 7;  // entries per record
 //          is kPruneSets lines, all 0 before the run.
 // field_bytes 1 (dwords 4, 8, 12, 16) or 2 (dwords 8, 16, 24).
 const void* int_prune_kernel_ptr(int field_bytes, int dwords, bool nodes);
+//   tables: (const int* blob, int field_bytes, int dwords, uint32_t* tables
+//          /* PrunePlan::lds_bytes */), 256 threads, a thread for every 4 bytes
+const void* prune_tables_kernel_ptr();
 constexpr int kPruneBlock = 512;
 constexpr int kPruneLevels = 12;      // column groups of 6 of 62 walked columns, and one
 constexpr int kPruneTopBits = 15;     // the first launch has at most 2^15 prefixes
