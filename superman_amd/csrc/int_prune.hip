@@ -3,9 +3,9 @@
 // out the matrix for it).
 //
 // What bounds it: VALU issue on the surviving nodes (about 5 instructions
-// per testable row and node of 4096 subsets) and terms (about 250
-// instructions per 64 terms at order 40); no memory but the tables (10 to 60
-// KB, once per block).
+// per testable row and node of 4096 subsets) and terms (at order 30 about 105
+// instructions per 64 terms and 9 for each round of the queue); no memory but
+// the tables (10 to 60 KB, once per block).  Half 0/1 order 30: 226 us.
 #include "walk_prune.h"
 
 namespace spm {
@@ -72,8 +72,12 @@ prune_tables_kernel(const int* __restrict__ blob, int field_bytes, int dwords, u
 // prefix that does not fit is walked depth first where it is found.  The
 // first launch has no list: its prefixes are all settings of the groups from
 // `group` + 1 (group 1: the nodes) outward, [begin, end), a power of two.
+//
+// 8 waves per SIMD where the registers allow it without spills to memory:
+// half 0/1 order 31 548 us, 580 at the 6 that the compiler's own scalar
+// registers leave.
 template <int FB, int NQ, bool NODES>
-__global__ void __launch_bounds__(kPruneBlock) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(kPruneBlock) __attribute__((amdgpu_waves_per_eu(NODES && FB == 1 && NQ <= 8 ? 8 : 4)))
 int_prune_kernel(const int* __restrict__ blob_, const uint4* __restrict__ tables,
                  const unsigned long long* __restrict__ in,
                  const unsigned int* __restrict__ in_count, unsigned long long* __restrict__ out,
@@ -82,6 +86,7 @@ int_prune_kernel(const int* __restrict__ blob_, const uint4* __restrict__ tables
 {
     constexpr int F = 4 / FB;
     constexpr int kWaves = kPruneBlock / kWave;
+    constexpr uint32_t kMany = 12;
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     __shared__ unsigned long long red[2 * kWaves];
     __shared__ unsigned long long stack[kWaves * kPruneLevels];
@@ -92,6 +97,26 @@ int_prune_kernel(const int* __restrict__ blob_, const uint4* __restrict__ tables
     const int nleaf = blob[kPruneLeaf], stride = blob[kPruneStride], mode = blob[kPruneMode];
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t w = uni(threadIdx.x / kWave);
+
+    // Prefixes are handed out in equal sets, one for every sets-th wave.
+    const uint32_t waves = gridDim.x * kWaves, wave = blockIdx.x * kWaves + w;
+    uint32_t sets = kPruneSets;
+    while (sets > waves) sets >>= 1;
+    const uint32_t set = wave & (sets - 1);
+    const uint32_t total = (uint32_t)(end - begin), share = max(1u, total / sets);
+    const uint32_t count = in_count ? min(uni(in_count[set * kPruneCounterStride]), cap) : set < total ? share : 0u;
+    // Runs of nodes, or batches of 64 prefixes whose settings are split over
+    // 2^cut waves where that leaves waves idle; `step`: waves of this set.
+    const uint32_t step = (waves - set + sets - 1) / sets;
+    const uint32_t run = max(1u, min(8u, count * sets / (waves * 8)));
+    const uint32_t batches = (count + kWave - 1) / kWave;
+    uint32_t cut = 0;
+    if (!NODES)
+        while (cut < 6 && (batches << cut) < 2 * step) ++cut;
+    if (!__syncthreads_or(wave / sets * (NODES ? run : 1u) < (NODES ? count : batches << cut))) {
+        if (threadIdx.x == 0) partial[2 * blockIdx.x] = partial[2 * blockIdx.x + 1] = 0;
+        return;  // no tables for nothing (order 28, 4 per row: 35 -> 28 us a run)
+    }
 
     uint32_t* tab = lds;
     unsigned long long* zt = (unsigned long long*)(lds + (size_t)G * 64 * NQ);
@@ -165,30 +190,48 @@ int_prune_kernel(const int* __restrict__ blob_, const uint4* __restrict__ tables
         if (!any) return;
         lo = ~lo;
         hi = ~hi;
-        const uint32_t first = tail;
-        for (;;) {
-            const bool has = (lo | hi) != 0;
-            const uint64_t m = __builtin_amdgcn_ballot_w64(has);
-            if (m == 0) break;
+        const uint32_t first = tail, plo = (uint32_t)prefix, phi = (uint32_t)(prefix >> 32);
+        // Subset `code` of the node into the queue, from each lane with `has`
+        // (m, their ballot).
+        auto push = [&](bool has, uint64_t m, uint32_t code) __attribute__((always_inline)) {
             const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)m, tail));
-            if (has) {
-                const bool low = lo != 0;
-                const uint32_t b = low ? (uint32_t)__builtin_ctz(lo) : 32u + (uint32_t)__builtin_ctz(hi);
-                if (low) lo &= lo - 1;
-                else hi &= hi - 1;
-                queue[at & (2 * kWave - 1)] = prefix | (lane << 6) | b;
-            }
+            if (has) queue[at & (2 * kWave - 1)] = ((uint64_t)phi << 32) | (plo | code);
             tail += (uint32_t)__builtin_popcountll(m);
             if (tail - head >= (uint32_t)kWave) flush(kWave, (int32_t)(head - first) >= 0, nb);
+        };
+        // A few lanes hold most of the subsets (half 0/1 order 30: 6 a lane,
+        // 28 the most).  A lane with many gives them all at once, setting by
+        // setting to the lanes; the others one each a round.
+        uint64_t many =
+            __builtin_amdgcn_ballot_w64((uint32_t)(__builtin_popcount(lo) + __builtin_popcount(hi)) > kMany);
+        if (many != 0) {
+            const uint32_t keep = (uint32_t)(__builtin_popcount(lo) + __builtin_popcount(hi)) > kMany ? 0u : ~0u;
+            do {
+                const int r = __builtin_ctzll(many);
+                many &= many - 1;
+                const uint64_t m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)hi, r) << 32) |
+                                   (uint32_t)__builtin_amdgcn_readlane((int)lo, r);
+                push(((m >> lane) & 1u) != 0, m, ((uint32_t)r << 6) | lane);
+            } while (many != 0);
+            lo &= keep;
+            hi &= keep;
+        }
+        uint32_t code = lane << 6;
+        uint32_t left = lo;
+        for (;;) {  // the words one after the other: 9 instructions a round, 16 for both as one word
+            const uint64_t m = __builtin_amdgcn_ballot_w64(left != 0);
+            if (m == 0) {
+                if (code & 32u) break;
+                code |= 32u;
+                left = hi;
+                continue;
+            }
+            push(left != 0, m, code | (uint32_t)__builtin_ctz(left));
+            left &= left - 1;
         }
     };
 
-    // Prefixes are handed out in equal sets, one for every sets-th wave.
-    const uint32_t waves = gridDim.x * kWaves, wave = blockIdx.x * kWaves + w;
-    uint32_t sets = kPruneSets;
-    while (sets > waves) sets >>= 1;
-    const uint32_t set = wave & (sets - 1);
     auto sums = [&](uint32_t (&c)[NQ], uint64_t prefix, int g) __attribute__((always_inline)) {  // groups >= g
 #pragma unroll
         for (int q = 0; q < NQ; ++q) c[q] = 0;
@@ -197,21 +240,22 @@ int_prune_kernel(const int* __restrict__ blob_, const uint4* __restrict__ tables
     // Prefix `id` of this set: from the list, or of all settings an odd
     // multiplier's spread, the set's own run of multiples (neighbouring
     // settings survive alike, and so do those that share their low bits).
-    const uint32_t total = (uint32_t)(end - begin), share = max(1u, total / sets);
-    const uint32_t count = in_count ? min(uni(in_count[set * kPruneCounterStride]), cap) : set < total ? share : 0u;
     auto prefix_of = [&](uint32_t id) __attribute__((always_inline)) {
         if (in_count) return (uint64_t)in[(size_t)set * cap + id];
         return (begin + (((set * share + id) * 0x9e3779b1u) & (total - 1))) << (6 * group + 6);
     };
     if constexpr (NODES) {
-        // Runs of nodes through a counter per set (the nodes' terms differ:
-        // an even share fixed beforehand ends 30 % later at half 0/1 order
-        // 32); the next run is fetched while one is walked, and one counter
-        // for all would cost 12 ns a fetch in atomics on one address.
+        // Runs of nodes, after each wave's first through a counter per set
+        // (the nodes' terms differ: an even share fixed beforehand ends 30 %
+        // later at half 0/1 order 32); the next run is fetched while one is
+        // walked, and one counter for all would cost 12 ns a fetch in atomics
+        // on one address.
         unsigned int* next_run = out_count + set * kPruneCounterStride;
-        const uint32_t run = max(1u, min(8u, count * sets / (waves * 8)));
-        uint32_t id = uni(atomicAdd(next_run, lane == 0 ? run : 0u));
-        uint32_t next = atomicAdd(next_run, lane == 0 ? run : 0u);
+        auto fetch = [&]() __attribute__((always_inline)) {  // past every wave's first run
+            return step * run + atomicAdd(next_run, lane == 0 ? run : 0u);
+        };
+        uint32_t id = wave / sets * run, next = 0;
+        if (id < count) next = fetch();
         while (id < count) {
             const uint32_t last = min(id + run, count);
             for (; id < last; ++id) {
@@ -222,12 +266,11 @@ int_prune_kernel(const int* __restrict__ blob_, const uint4* __restrict__ tables
                 node(nb, prefix);
             }
             id = uni(next);
-            if (id < count) next = atomicAdd(next_run, lane == 0 ? run : 0u);
+            if (id < count) next = fetch();
         }
     } else {
         unsigned int* listed = out_count + set * kPruneCounterStride;
         unsigned long long* seg = out + (size_t)set * cap;
-        const uint32_t step = (waves - set + sets - 1) / sets;  // waves of this set
         uint32_t cur[NQ];  // packed sums of the groups set so far
         uint64_t left = 0;  // settings of group g still to visit
         int g = group;
@@ -284,9 +327,6 @@ int_prune_kernel(const int* __restrict__ blob_, const uint4* __restrict__ tables
         // settings are split over 2^cut of them.
         const uint32_t used = (uint32_t)blob[kPruneUsed + group];
         const const_i32* care = blob + prune_care_at(NQ, NQ * F) + group * NQ;
-        const uint32_t batches = (count + kWave - 1) / kWave;
-        uint32_t cut = 0;
-        while (cut < 6 && (batches << cut) < 2 * step) ++cut;
         for (uint32_t u = wave / sets; u < (batches << cut); u += step) {
             const uint32_t id = (u >> cut) * kWave + lane, each = 64u >> cut;
             bool valid = id < count;

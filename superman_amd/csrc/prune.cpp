@@ -176,20 +176,28 @@ bool prune_plan(const int64_t* a, int n, const unsigned char* w, PrunePlan& p)
     p.first_group = t;
     p.prefixes = uint64_t(1) << (B - 6 * t);
 
-    // Exact product groups: bits of each aligned run of fields.
-    auto run_bits = [&](int len) {
+    // Exact product groups: bits of the rows' values in runs of `len` fields
+    // at i and i + half (0: none).
+    auto run_bits = [&](int len, int half) {
         double worst = 0;
-        for (int i = 0; i < fields; i += len) {
+        for (int i = 0; i < (half ? half : fields); i += len) {
             double s = 0;
             for (int k = i; k < i + len; ++k)
-                s += std::log2((double)std::max(1, std::max(std::abs(rows[k].o), std::abs(rows[k].o + rows[k].width))));
+                for (int j = k; j < fields; j += half ? half : fields)
+                    s += std::log2(
+                        (double)std::max(1, std::max(std::abs(rows[j].o), std::abs(rows[j].o + rows[j].width))));
             worst = std::max(worst, s);
         }
         return worst;
     };
     int mode = 0;
-    if (fb == 1) mode = run_bits(8) < 30.9 ? 2 : run_bits(4) < 30.9 ? 1 : 0;
-    else mode = run_bits(4) < 62.9 ? 1 : 0;
+    if (fb == 1) {
+        bool bytes = true;
+        for (const Row& r : rows) bytes = bytes && r.o >= -128 && r.o + r.width <= 127;
+        mode = !bytes ? 0 : run_bits(8, fields / 2) < 62.9 ? 2 : 1;
+    } else {
+        mode = run_bits(4, 0) < 62.9 ? 1 : 0;
+    }
 
     std::vector<int>& b = p.blob;
     b.assign(prune_blob_ints(nq, fields), 0);
@@ -197,7 +205,10 @@ bool prune_plan(const int64_t* a, int n, const unsigned char* w, PrunePlan& p)
         v[field / F] = (int)((uint32_t)v[field / F] + (x << (8 * fb * (field % F))));
     };
     int* o = b.data() + prune_offset_at(nq);
-    for (int i = 0; i < fields; ++i) o[i] = rows[i].o;
+    for (int i = 0; i < fields; ++i) {
+        if (fb == 1 && mode != 0) put(o, i, (uint32_t)(rows[i].o + 128));
+        else o[i] = rows[i].o;
+    }
     for (int i = 0; i < fields; ++i)
         if (rows[i].test) put(b.data() + kPruneZero, i, (uint32_t)-rows[i].o);
     int* care = b.data() + prune_care_at(nq, fields);
@@ -228,16 +239,16 @@ bool prune_plan(const int64_t* a, int n, const unsigned char* w, PrunePlan& p)
 }
 
 // Whether the pruned walk is the faster one.  Its time, fitted to kernel
-// times at orders 24-48: 15 us and 20 us a launch (tables, launch gap), 0.55
-// ns a node and 8e-12 (n + 40) / 70 s a surviving term, against the walks'
-// rates (int_walk_costs, launches 15 us).  Measured on both sides of the
-// line: half 0/1 order 26 0.12 against 0.12 ms (FP64 walk), order 30 0.39
-// against 1.51, order 24 with 4 entries per row 0.060 against 0.038, order
-// 28 0.063 against 0.14 (compressed columns), order 40 0.12 against 229; with
-// odd row sums throughout every term survives (order 26 0.18 against 0.12).
-// The row-independence estimate of the surviving share runs low where rows
-// are alike, so nodes and terms count double, and from order 30, where a
-// wrong choice costs milliseconds, a sample of the subsets has a say.
+// times at orders 24-48: 18 us and 8 us a launch, 0.4 ns a node and 4.8e-12
+// (n + 40) / 70 s a surviving term, against the walks' rates (int_walk_costs,
+// launches 15 us).  Measured on both sides of the line, pruned against the
+// best walk: half 0/1 order 24 57 against 39 us, order 25 58 against 61, order
+// 28 0.14 against 0.37 ms; 3 per row (every term survives) order 26 130
+// against 105 us, order 28 0.42 against 0.38 ms; 4 per row order 25 26 against
+// 37 us.  (90 % ones order 30 is left to the FP64 walk: 1.49 against 1.08 ms.)
+// The row-independence estimate of the surviving share runs low where rows are
+// alike, so nodes and terms count double; from order 30, where a wrong choice
+// costs milliseconds, a sample of the subsets says.
 bool prune_preferred(const int64_t* a, int n, const PrunePlan& p)
 {
     const IntWalkCosts c = int_walk_costs(a, n);
@@ -262,12 +273,12 @@ bool prune_preferred(const int64_t* a, int n, const PrunePlan& p)
             }
             nonzero += nz ? 1 : 0;
         }
-        q = std::max(q, double(nonzero) / kSamples);
+        q = std::min(1.0, 1.25 * std::max(c.q, double(nonzero) / kSamples));
     }
     const double subsets = std::ldexp(1.0, n - 1);
-    const double pruned = 1.5e-5 + 2e-5 * (p.first_group - 1) +
-                          5.5e-10 * std::min(2.0 * p.nodes, std::ldexp(1.0, n - 13)) +
-                          q * subsets * 8e-12 * (n + 40) / 70.0;
+    const double pruned = 1.8e-5 + 8e-6 * (p.first_group - 1) +
+                          4e-10 * std::min(2.0 * p.nodes, std::ldexp(1.0, n - 13)) +
+                          q * subsets * 4.8e-12 * (n + 40) / 70.0;
     const double walk = n >= 26 ? std::min(c.sparse, std::min(c.fp64, c.int32)) : std::min(c.fp64, c.int32);
     return pruned < 1.5e-5 + subsets * walk;
 }

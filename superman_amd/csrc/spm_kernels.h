@@ -127,7 +127,7 @@ enum PruneSlot {
     kPruneUsed = 8,                               // [kPruneLevels] dwords with a nonzero care mask
     kPruneZero = kPruneUsed + kPruneLevels        // [dwords] packed zero pattern, -o; then:
 };
-constexpr int prune_offset_at(int dwords) { return kPruneZero + dwords; }              // [fields] o: y = field + o
+constexpr int prune_offset_at(int dwords) { return kPruneZero + dwords; }              // [fields] o: y = field + o (or packed, product())
 constexpr int prune_care_at(int dwords, int fields) { return prune_offset_at(dwords) + fields; }  // [kPruneLevels][dwords]
 constexpr int prune_on_at(int dwords, int fields)     // [kMaxN][2][dwords] a column's fields: in the subset, out of it
 {
