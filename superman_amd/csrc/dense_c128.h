@@ -22,6 +22,7 @@ __device__ __forceinline__ void c128_chunks(const double* __restrict__ M, const 
     // Only a grid with fewer than 64 chunks has idle lanes, and then each
     // lane has exactly one task: such lanes' sums are dropped at the end.
     const bool idle = (uint64_t)lane >= num_chunks;
+    touch_lines<4 * N * N, kDenseBlock>(M, threadIdx.x);
     double re_hi = 0.0, re_lo = 0.0, im_hi = 0.0, im_lo = 0.0, abs_sum = 0.0;
 
     for (uint64_t task = task_begin + wave; task < task_end; task += nwave) {

@@ -30,6 +30,7 @@ int_dense_kernel(const int* __restrict__ M,        // [2][N][N]: +2A then -2A, c
     const uint64_t wave = (uint64_t)blockIdx.x * (kDenseBlock / kWave) + (threadIdx.x / kWave);
     const uint64_t nwave = (uint64_t)gridDim.x * (kDenseBlock / kWave);
     const bool idle = (uint64_t)lane >= num_chunks;  // see dense_c128.hip
+    touch_lines<N * N, kDenseBlock>((const double*)M, threadIdx.x);
     unsigned __int128 acc = 0;
 
     for (uint64_t task = task_begin + wave; task < task_end; task += nwave) {

@@ -13,6 +13,13 @@ namespace spm {
 
 constexpr int kWave = 64;
 
+// The first active lane's value, as a scalar.
+__device__ __forceinline__ uint64_t wave_bits(uint64_t v)
+{
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+           (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+}
+
 // TwoSum (Knuth): s + e == a + b exactly.
 __device__ __forceinline__ void two_sum(double a, double b, double& s, double& e)
 {
@@ -84,6 +91,24 @@ __device__ __forceinline__ void block_reduce_dd(double& hi, double& lo, double& 
         lo = l;
         ab = a;
     }
+}
+
+// Threads 0..THREADS-1 (this one is t) read every line of M[0, DOUBLES) once.
+// A freshly uploaded matrix is in none of this die's caches, and a walk starts
+// with a chain of scalar loads, a column each, that would miss one after the
+// other (about 0.7 us a column: a call at complex order 21 57 -> 39 us).
+template <int DOUBLES, int THREADS>
+__device__ __forceinline__ void touch_lines(const double* M, uint32_t t)
+{
+    constexpr int kLines = (DOUBLES + 15) / 16, kEach = (kLines + THREADS - 1) / THREADS;
+    double v[kEach];
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) {
+        const uint32_t line = t + (uint32_t)(i * THREADS);
+        v[i] = M[16 * (line < (uint32_t)kLines ? line : 0u)];
+    }
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) asm volatile("" ::"v"(v[i]));
 }
 
 }  // namespace spm

@@ -331,10 +331,13 @@ __device__ __forceinline__ void walk_c128(const double* __restrict__ M,   // [2]
     stream_column<N, 0>(x, x0, 0.0);
     const uint64_t k0 = h << L;
     const uint64_t g0 = k0 ^ (k0 >> 1);
-    for (int j = (L > 0 ? L - 1 : 0); j < NC; ++j) {
+    const int shared = min(NC, L + 6);  // columns from here on: set for the whole wave or not
+    for (int j = (L > 0 ? L - 1 : 0); j < shared; ++j) {
         const double b = ((g0 >> j) & 1u) ? 1.0 : 0.0;
         stream_column<N, 2>(x, M + (size_t)j * C, b);
     }
+    for (uint64_t left = wave_bits(g0) & ((uint64_t(1) << NC) - (uint64_t(1) << shared)); left != 0; left &= left - 1)
+        stream_column<N, 2>(x, M + (size_t)__builtin_ctzll(left) * C, 1.0);
 
     const double lane_sign = (h & 1u) ? -1.0 : 1.0;
     double br = 0.0, bi = 0.0, babs = 0.0;

@@ -115,11 +115,18 @@ __device__ __forceinline__ void walk_int(const int* __restrict__ M,   // [2][N][
     }
     const uint64_t k0 = h << L;
     const uint64_t g0 = k0 ^ (k0 >> 1);
-    for (int j = (L > 0 ? L - 1 : 0); j < N - 1; ++j) {
+    const int shared = min(N - 1, L + 6);  // columns from here on: set for the whole wave or not
+    for (int j = (L > 0 ? L - 1 : 0); j < shared; ++j) {
         const int b = -(int)((g0 >> j) & 1u);  // 0 or -1: mask of "column j in the start set"
         const const_i32* __restrict__ col = step_ptr(M + j * N);
 #pragma unroll
         for (int r = 0; r < N; ++r) y[r] += col[r] & b;
+    }
+    for (uint64_t left = wave_bits(g0) & ((uint64_t(1) << (N - 1)) - (uint64_t(1) << shared)); left != 0;
+         left &= left - 1) {
+        const const_i32* __restrict__ col = step_ptr(M + __builtin_ctzll(left) * N);
+#pragma unroll
+        for (int r = 0; r < N; ++r) y[r] += col[r];
     }
     const int lane_mask = -(int)(h & 1u);  // direction of column L-1: -1 = remove
 
