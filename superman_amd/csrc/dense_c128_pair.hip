@@ -3,8 +3,8 @@
 // subsets per step (PairProd in walk_c128.h).
 //
 // VALU issue bounds it: 162 FP64 instructions per subset at order 32 (191 in
-// dense_c128_kernel); Haar order 32 takes 10.76 ms a call (12.86 there), Gauss
-// order 24 54 us of kernel (62), order 30 2.53 ms (2.91).
+// dense_c128_kernel); Haar order 32 takes 10.5-10.8 ms a call (12.7 there),
+// Gauss order 24 52 us a run (62), order 30 2.41 ms (2.91).
 #include "dense_c128.h"
 
 // SPM_C128_ONLY_N (sweeps only): instantiate a single order.

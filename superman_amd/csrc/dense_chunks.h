@@ -21,7 +21,7 @@ __device__ __forceinline__ void dense_chunks(const double* __restrict__ M, const
     const uint64_t wave = (uint64_t)blockIdx.x * (kDenseBlock / kWave) + (threadIdx.x / kWave);
     const uint64_t nwave = (uint64_t)gridDim.x * (kDenseBlock / kWave);
 
-    touch_lines<2 * N * N, kDenseBlock>(M, threadIdx.x);
+    touch_lines<(N + 1 + NC) * N, kDenseBlock>(M, threadIdx.x);  // M is column N - 1 - NC of the first plane
     double acc_hi = 0.0, acc_lo = 0.0, acc_abs = 0.0;
     for (uint64_t task = task_begin + wave; task < task_end; task += nwave) {
         const uint64_t h = task * kWave + lane;

@@ -4,7 +4,7 @@
 //
 // VALU issue bounds it: 62.5 FP64 instructions per subset at order 40 (80.8
 // in dense_f64_kernel), no memory traffic to speak of; order 40 takes 1013 ms
-// (1269 ms there), order 33 plain 6.7 ms (8.15 ms).  That is 4.6 cycles per
+// (1269 ms there), order 33 plain 6.3 ms (8.0 ms).  That is 4.6 cycles per
 // wave instruction; a loop of such multiplies and FMAs alone takes 4.5 at the
 // same 4 waves per SIMD.  127 VGPRs at order 40 allow no fifth wave, and
 // asking for 5 at orders 25-38 or 6 below moved no time by more than 2 %.

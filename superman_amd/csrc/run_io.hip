@@ -3,7 +3,7 @@
 // memory, and the reduced sums back into pinned memory behind a flag the host
 // polls.  With the plan's memory from a pool (workspace.cpp) a call then makes
 // no allocation, no copy command and no stream synchronization: order 8 from
-// 77-97 to 26 us a call, of which 9 us are three launches and a flag.
+// 77-97 to 20 us a call, of which 9 us are three launches and a flag.
 #include "dense_reduce.h"
 #include "spm_kernels.h"
 
