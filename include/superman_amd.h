@@ -185,8 +185,11 @@ int spm_plan_int(const int64_t* a, int n, int device, spm_plan** plan);
  * per step only the flipped column's rows, a zero-row count, the product
  * only when no row is zero; the reference's runtime-CSC sparse kernels,
  * SparseKernelDefinitions.cuh:34-509) or SPM_INT_WALK_PRUNED (only the
- * subsets with no zero row, found by a search over column groups; n >= 13
- * and 2 sum_j |a_ij| below 2^16 for every row, else SPM_ERANGE).
+ * subsets with no zero row, found by a search over column groups; n >= 13,
+ * and packed row sums: in 8 bits when 2 sum_j |a_ij| <= 255 in every row, up
+ * to order 43 in 16 bits when that is below 2^16; the sums leave out one
+ * column of the plan's choice, whose entries may be larger where the products
+ * of two rows still fit 32 bits or the order is at most 43; else SPM_ERANGE).
  * SPM_INT_WALK_AUTO takes the one with the lowest estimated time. */
 #define SPM_INT_WALK_AUTO   0
 #define SPM_INT_WALK_INT32  1

@@ -86,56 +86,23 @@ std::vector<int> inner_first_order(const std::vector<uint64_t>& rows_of, const s
     return best;
 }
 
-}  // namespace
+// A row's bounds in the plan's column order: field = sum of positive entries
+// in S and of |negative| entries outside S (times w), y = field + o.  The
+// last column is in no subset: its entry is in o alone, which can be far
+// larger than the field.
+struct Row {
+    int src, low, o, width, outer;
+    bool test;
+};
 
-bool prune_plan(const int64_t* a, int n, const unsigned char* w, PrunePlan& p)
+// The layout with fields of fb bytes.  False when it has no kernel, its tables
+// do not fit, or 8-bit fields leave a product that product() would not form
+// exactly.
+bool lay_out(const int64_t* a, int n, const unsigned char* w, const std::vector<int>& ord, std::vector<Row> rows, int fb,
+             PrunePlan& p)
 {
-    if (n < kPruneMinN || n > kMaxN) return false;
     const int B = n - 1, G = (B + 5) / 6;
-
-    std::vector<double> bits(n, 0.0);
-    std::vector<uint64_t> rows_of(n, 0);
-    for (int i = 0; i < n; ++i) {
-        int k = 0;
-        for (int j = 0; j < n; ++j) k += a[(size_t)i * n + j] != 0 ? 1 : 0;
-        if (w[i] != 1) continue;  // an odd row sum: never zero
-        bits[i] = row_bits(k);
-        for (int j = 0; j < n; ++j)
-            if (a[(size_t)i * n + j] != 0) rows_of[j] |= uint64_t(1) << i;
-    }
-    double nodes = 0, upper = 0;
-    const std::vector<int> ord = inner_first_order(rows_of, bits, n, &nodes, &upper);
-
-    // Row bounds in this order: field = sum of positive entries in S and of
-    // |negative| entries outside S (times w), y = field + o.
-    struct Row {
-        int src, low, o, width, outer;
-        bool test;
-    };
-    std::vector<Row> rows(n);
-    int64_t widest = 0;
-    for (int i = 0; i < n; ++i) {
-        Row& r = rows[i];
-        int64_t sum = 0, width = 0, neg = 0, inner = 0;
-        r.src = i;
-        r.low = G;
-        for (int j = 0; j < n; ++j) sum += a[(size_t)i * n + j];
-        for (int k = 0; k < B; ++k) {
-            const int64_t v = w[i] * a[(size_t)i * n + ord[k]], m = v < 0 ? -v : v;
-            width += m;
-            if (v < 0) neg += m;
-            if (k < 6) inner += m;
-            if (v != 0) r.low = std::min(r.low, k / 6);
-        }
-        const int64_t y0 = (2 * a[(size_t)i * n + ord[B]] - sum) / (w[i] == 1 ? 2 : 1);
-        widest = std::max(widest, width);
-        if (width > 0xffff) return false;
-        r.o = (int)(y0 - neg);
-        r.width = (int)width;
-        r.outer = (int)(width - inner);
-        r.test = w[i] == 1 && -r.o >= 0 && -r.o <= r.width;
-    }
-    const int fb = widest <= 0xff ? 1 : 2, F = 4 / fb;
+    const int F = 4 / fb;
     const int nq = fb == 1 ? 4 * ((n + 15) / 16) : 8 * ((n + 15) / 16);
     if (fb == 2 && nq > 24) return false;
 
@@ -178,14 +145,15 @@ bool prune_plan(const int64_t* a, int n, const unsigned char* w, PrunePlan& p)
 
     // Exact product groups: bits of the rows' values in runs of `len` fields
     // at i and i + half (0: none).
+    auto top = [&](int i) {  // the largest |y|
+        return std::max<int64_t>(1, std::max(std::abs((int64_t)rows[i].o), std::abs((int64_t)rows[i].o + rows[i].width)));
+    };
     auto run_bits = [&](int len, int half) {
         double worst = 0;
         for (int i = 0; i < (half ? half : fields); i += len) {
             double s = 0;
             for (int k = i; k < i + len; ++k)
-                for (int j = k; j < fields; j += half ? half : fields)
-                    s += std::log2(
-                        (double)std::max(1, std::max(std::abs(rows[j].o), std::abs(rows[j].o + rows[j].width))));
+                for (int j = k; j < fields; j += half ? half : fields) s += std::log2((double)top(j));
             worst = std::max(worst, s);
         }
         return worst;
@@ -195,6 +163,10 @@ bool prune_plan(const int64_t* a, int n, const unsigned char* w, PrunePlan& p)
         bool bytes = true;
         for (const Row& r : rows) bytes = bytes && r.o >= -128 && r.o + r.width <= 127;
         mode = !bytes ? 0 : run_bits(8, fields / 2) < 62.9 ? 2 : 1;
+        // two rows of a dword multiply in 32 bits (fours of such pairs then
+        // fit 64); 16-bit fields form every product in 64
+        for (int i = 0; mode == 0 && i < fields; i += 2)
+            if (top(i) * top(i + 1) > INT32_MAX) return false;
     } else {
         mode = run_bits(4, 0) < 62.9 ? 1 : 0;
     }
@@ -233,9 +205,55 @@ bool prune_plan(const int64_t* a, int n, const unsigned char* w, PrunePlan& p)
     p.field_bytes = fb;
     p.dwords = nq;
     p.lds_bytes = (int)(table + (size_t)nleaf * stride * 8);
+    return true;
+}
+
+}  // namespace
+
+bool prune_plan(const int64_t* a, int n, const unsigned char* w, PrunePlan& p)
+{
+    if (n < kPruneMinN || n > kMaxN) return false;
+    const int B = n - 1, G = (B + 5) / 6;
+
+    std::vector<double> bits(n, 0.0);
+    std::vector<uint64_t> rows_of(n, 0);
+    for (int i = 0; i < n; ++i) {
+        int k = 0;
+        for (int j = 0; j < n; ++j) k += a[(size_t)i * n + j] != 0 ? 1 : 0;
+        if (w[i] != 1) continue;  // an odd row sum: never zero
+        bits[i] = row_bits(k);
+        for (int j = 0; j < n; ++j)
+            if (a[(size_t)i * n + j] != 0) rows_of[j] |= uint64_t(1) << i;
+    }
+    double nodes = 0, upper = 0;
+    const std::vector<int> ord = inner_first_order(rows_of, bits, n, &nodes, &upper);
+
+    std::vector<Row> rows(n);
+    int64_t widest = 0;
+    for (int i = 0; i < n; ++i) {
+        Row& r = rows[i];
+        int64_t sum = 0, width = 0, neg = 0, inner = 0;
+        r.src = i;
+        r.low = G;
+        for (int j = 0; j < n; ++j) sum += a[(size_t)i * n + j];
+        for (int k = 0; k < B; ++k) {
+            const int64_t v = w[i] * a[(size_t)i * n + ord[k]], m = v < 0 ? -v : v;
+            width += m;
+            if (v < 0) neg += m;
+            if (k < 6) inner += m;
+            if (v != 0) r.low = std::min(r.low, k / 6);
+        }
+        const int64_t y0 = (2 * a[(size_t)i * n + ord[B]] - sum) / (w[i] == 1 ? 2 : 1);
+        widest = std::max(widest, width);
+        if (width > 0xffff) return false;
+        r.o = (int)(y0 - neg);
+        r.width = (int)width;
+        r.outer = (int)(width - inner);
+        r.test = w[i] == 1 && -r.o >= 0 && -r.o <= r.width;
+    }
     p.nodes = nodes;
     p.upper = upper;
-    return true;
+    return (widest <= 0xff && lay_out(a, n, w, ord, rows, 1, p)) || lay_out(a, n, w, ord, rows, 2, p);
 }
 
 // Whether the pruned walk is the faster one.  Its time, fitted to kernel

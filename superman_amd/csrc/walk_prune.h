@@ -99,7 +99,8 @@ __device__ __forceinline__ bool rows_nonzero(const uint32_t (&c)[NQ], const int*
 
 // prod_i y_i mod 2^128 of one subset's packed sums, y = field + o (padding
 // fields are 0 with o = 1).  The host picks `mode` from the rows' bounds:
-//   8-bit fields:  0: any y; 2 rows multiply exactly in 32 bits, 4 in 64.
+//   8-bit fields:  0: two rows of a dword multiply exactly in 32 bits, 4 in 64
+//     (the host lays a matrix with larger |y| out in 16-bit fields).
 //     1: every y is a signed byte; the offset section holds o + 128 packed,
 //     and with the top bits flipped the sums are the y themselves, which the
 //     multiplier takes as they are (a byte select is part of the instruction):
@@ -108,7 +109,7 @@ __device__ __forceinline__ bool rows_nonzero(const uint32_t (&c)[NQ], const int*
 //     that can be zero come first and are carried halved).
 //     With offsets added row by row (5 instead of 1 instructions for two
 //     rows) half 0/1 order 30 took 294 instead of 247 us.
-//   16-bit fields: 0: 1 row in 32 bits, 2 in 64;  1: 1 and 4
+//   16-bit fields: 0: any |y| < 2^30, 1 row in 32 bits, 2 in 64;  1: 1 and 4
 template <int FB, int NQ>
 __device__ __forceinline__ unsigned __int128 product(const uint32_t (&c)[NQ], const int* blob_, int mode)
 {
