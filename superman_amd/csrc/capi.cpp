@@ -795,7 +795,8 @@ extern "C" int spm_codegen_source_real(const double* a, int n, int options, int 
     if (rc != SPM_OK) return rc;
     const std::vector<double> b = codegen_matrix_real(a, n, options);
     const std::string src = emit_real_kernel(b, n, precision == SPM_PREC_COMPENSATED,
-                                             codegen_real_name(real_pattern_hash(b.data(), n, options, precision)));
+                                             codegen_real_name(real_pattern_hash(b.data(), n, options, precision)),
+                                             real_elim_columns(b.data(), n));
     if (needed) *needed = src.size() + 1;
     if (buf && buflen > 0) {
         const size_t k = std::min(buflen - 1, src.size());
@@ -827,9 +828,10 @@ extern "C" int spm_plan_codegen_real(const double* a, int n, int options, int pr
     p->comps = 1;
     p->hash = real_pattern_hash(b.data(), n, options, precision);
     p->kname = codegen_real_name(p->hash);
+    const int elim = real_elim_columns(b.data(), n);
     rc = codegen_get_kernel(device, p->hash,
-                            emit_real_kernel(b, n, precision == SPM_PREC_COMPENSATED, p->kname), p->kname, &p->fn,
-                            &p->compile_s, &p->cached);
+                            emit_real_kernel(b, n, precision == SPM_PREC_COMPENSATED, p->kname, elim), p->kname,
+                            &p->fn, &p->compile_s, &p->cached);
     if (rc != SPM_OK) {
         plan_free(p);
         return rc;
@@ -841,11 +843,11 @@ extern "C" int spm_plan_codegen_real(const double* a, int n, int options, int pr
     }
     const int64_t waves = int64_t(bpc) * cus * (kDenseBlock / kWaveLanes);
     gray_geometry(n, codegen_real_unroll_bits(n), waves, &p->L, &p->chunks, &p->tasks);
-    if (const int m = real_elim_columns(b.data(), n)) {
+    if (elim > 0) {
         // 4 to 64 outer steps per chunk, two chunks or more per lane
         int lw = 0;
         while ((int64_t(1) << lw) < waves) ++lw;
-        p->L = m + std::min(6, std::max(2, n - 1 - m - 6 - lw - 1));
+        p->L = elim + std::min(6, std::max(2, n - 1 - elim - 6 - lw - 1));
         p->chunks = uint64_t(1) << (n - 1 - p->L);
         p->tasks = (p->chunks + kWaveLanes - 1) / kWaveLanes;
     }

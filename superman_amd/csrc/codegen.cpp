@@ -649,11 +649,15 @@ class Eliminator {
 public:
     Eliminator(const std::vector<double>& b, int n, int m) : b_(b), n_(n), m_(m) {}
 
-    // Emits E into `P` and its absolute sum into `A`.  False when an inner
-    // column is empty.  ops: FP64 instructions; peak: table entries alive.
-    bool run(int& ops, int& peak, std::string* code, const char* ind)
+    // Emits E into `P` and its absolute sum into `A`; without `code` it only
+    // counts.  False when an inner column is empty, or as soon as the code
+    // passes max_ops instructions or the tables max_peak values.  ops: FP64
+    // instructions; peak: table entries alive.
+    bool run(int& ops, int& peak, int max_ops, int max_peak, std::string* code = nullptr, const char* ind = "")
     {
         ops = peak = 0;
+        max_ops_ = max_ops;
+        emit_ = code != nullptr;
         ind_ = ind;
         std::vector<Factor> fs;
         for (int r = 0; r < n_; ++r) {
@@ -681,7 +685,7 @@ public:
             left.erase(left.begin() + pick);
             std::vector<Factor> with, rest;
             for (Factor& f : fs) {
-                if (has(f, c)) write_row(f, ops);
+                if (has(f, c) && !write_row(f, ops)) return false;
                 (has(f, c) ? with : rest).push_back(std::move(f));
             }
             while (with.size() > 2) {  // the pair with the smallest common scope first
@@ -695,25 +699,28 @@ public:
                             bj = j;
                         }
                     }
-                Factor f = multiply(with[bj], with[bi], ops);
+                Factor f;
+                if (!multiply(with[bj], with[bi], ops, f)) return false;
                 with.erase(with.begin() + bi);
                 with[bj] = std::move(f);
             }
-            rest.push_back(sum_out(with, c, ops));
+            rest.emplace_back();
+            if (!sum_out(with, c, ops, rest.back())) return false;
             fs = std::move(rest);
             int alive = 0;
             for (const Factor& f : fs) alive += (f.pure ? 1 : 2) * (int)f.val.size();  // (unwritten rows: none)
             peak = std::max(peak, alive);
-            if (peak > 1024) return false;
+            if (peak > max_peak) return false;
         }
+        ops += 2 * (int)fs.size();
+        if (ops > max_ops || !code) return ops <= max_ops;
         std::string P, A;
         for (const Factor& f : fs) {
             P += (P.empty() ? "" : " * ") + f.val[0];
             A += (A.empty() ? "" : " * ") + f.abs[0];
-            ops += 2;
         }
         line("const double P = " + P + ", A = " + A + ";");
-        if (code) *code = out_.str();
+        *code = out_.str();
         return true;
     }
 
@@ -738,52 +745,77 @@ private:
     void line(const std::string& t) { out_ << ind_ << t << "\n"; }
     std::string fresh(const char* stem) { return stem + std::to_string(id_++); }
     static std::string fabs(const std::string& v) { return "__builtin_fabs(" + v + ")"; }
-
-    void write_row(Factor& f, int& ops)
+    // `count` more instructions, if they are within the limit: asked before a
+    // table is written, which has 2^scope entries (rows of 40 entries at m = 16
+    // spelled out took 8 s and 0.5 GB before the limits were looked at).
+    bool take(int& ops, size_t count)
     {
-        if (f.row < 0) return;
-        f.val.push_back("x" + std::to_string(f.row));
-        for (size_t k = 0; k < f.scope.size(); ++k)
-            for (size_t i = 0, end = size_t(1) << k; i < end; ++i) {
-                const std::string v = fresh("v");
-                line("const double " + v + " = " + f.val[i] + " + " + hexlit(b_[(size_t)f.row * n_ + f.scope[k]]) + ";");
-                f.val.push_back(v);
-                ++ops;
-            }
-        for (const std::string& v : f.val) f.abs.push_back(fabs(v));
-        f.row = -1;
+        if (count > (size_t)(max_ops_ - ops)) return false;
+        ops += (int)count;
+        return true;
     }
-    Factor multiply(const Factor& f, const Factor& g, int& ops)
+
+    bool write_row(Factor& f, int& ops)
     {
-        Factor h;
+        if (f.row < 0) return true;
+        const size_t entries = size_t(1) << f.scope.size();
+        if (!take(ops, entries - 1)) return false;
+        if (emit_) {
+            f.val.push_back("x" + std::to_string(f.row));
+            for (size_t k = 0; k < f.scope.size(); ++k)
+                for (size_t i = 0, end = size_t(1) << k; i < end; ++i) {
+                    const std::string v = fresh("v");
+                    line("const double " + v + " = " + f.val[i] + " + " + hexlit(b_[(size_t)f.row * n_ + f.scope[k]]) +
+                         ";");
+                    f.val.push_back(v);
+                }
+            for (const std::string& v : f.val) f.abs.push_back(fabs(v));
+        } else {
+            f.val.resize(entries);
+        }
+        f.row = -1;
+        return true;
+    }
+    bool multiply(const Factor& f, const Factor& g, int& ops, Factor& h)
+    {
         h.scope = unite(f.scope, g.scope);
         h.pure = f.pure && g.pure;
-        for (size_t i = 0; i < size_t(1) << h.scope.size(); ++i) {
+        const size_t entries = size_t(1) << h.scope.size();
+        if (!take(ops, (h.pure ? 1 : 2) * entries)) return false;
+        if (!emit_) {
+            h.val.resize(entries);
+            return true;
+        }
+        for (size_t i = 0; i < entries; ++i) {
             const size_t fi = project(f, h.scope, i), gi = project(g, h.scope, i);
             const std::string v = fresh("p");
             line("const double " + v + " = " + f.val[fi] + " * " + g.val[gi] + ";");
             h.val.push_back(v);
-            ++ops;
             if (h.pure) {
                 h.abs.push_back(fabs(v));
             } else {
                 const std::string u = fresh("q");
                 line("const double " + u + " = " + f.abs[fi] + " * " + g.abs[gi] + ";");
                 h.abs.push_back(u);
-                ++ops;
             }
         }
-        return h;
+        return true;
     }
-    Factor sum_out(const std::vector<Factor>& fs, int c, int& ops)
+    bool sum_out(const std::vector<Factor>& fs, int c, int& ops, Factor& h)
     {
         const std::vector<int> scope = fs.size() == 2 ? unite(fs[0].scope, fs[1].scope) : fs[0].scope;
         const size_t at = std::lower_bound(scope.begin(), scope.end(), c) - scope.begin();
-        Factor h;
+        const bool pure = fs.size() == 2 && fs[0].pure && fs[1].pure;
         h.pure = false;
         for (int s : scope)
             if (s != c) h.scope.push_back(s);
-        for (size_t i = 0; i < size_t(1) << h.scope.size(); ++i) {
+        const size_t entries = size_t(1) << h.scope.size();
+        if (!take(ops, (fs.size() == 1 ? 2 : pure ? 3 : 4) * entries)) return false;
+        if (!emit_) {
+            h.val.resize(entries);
+            return true;
+        }
+        for (size_t i = 0; i < entries; ++i) {
             const size_t i0 = ((i >> at) << (at + 1)) | (i & ((size_t(1) << at) - 1)), i1 = i0 | (size_t(1) << at);
             const std::string v = fresh("t"), u = fresh("u");
             const Factor& f = fs[0];
@@ -791,7 +823,6 @@ private:
             if (fs.size() == 1) {
                 line("const double " + v + " = " + f.val[f0] + " - " + f.val[f1] + ";");
                 line("const double " + u + " = " + f.abs[f0] + " + " + f.abs[f1] + ";");
-                ops += 2;
             } else {
                 const Factor& g = fs[1];
                 const size_t g0 = project(g, scope, i0), g1 = project(g, scope, i1);
@@ -799,23 +830,23 @@ private:
                 line("const double " + p + " = " + f.val[f0] + " * " + g.val[g0] + ";");
                 line("const double " + v + " = __builtin_fma(-" + f.val[f1] + ", " + g.val[g1] + ", " + p + ");");
                 std::string q = fabs(p);
-                ops += 3;
-                if (!f.pure || !g.pure) {
+                if (!pure) {
                     q = fresh("q");
                     line("const double " + q + " = " + f.abs[f0] + " * " + g.abs[g0] + ";");
-                    ++ops;
                 }
                 line("const double " + u + " = __builtin_fma(" + f.abs[f1] + ", " + g.abs[g1] + ", " + q + ");");
             }
             h.val.push_back(v);
             h.abs.push_back(u);
         }
-        return h;
+        return true;
     }
 
     const std::vector<double>& b_;
     int n_, m_;
     const char* ind_ = "";
+    bool emit_ = false;
+    int max_ops_ = 0;
     int id_ = 0;
     std::ostringstream out_;
 };
@@ -847,6 +878,8 @@ static void emit_real_tail(std::ostringstream& o)
          "}\n";
 }
 
+constexpr int kElimOps = 1000, kElimPeak = 128;
+
 // The number m of inner columns to sum out: the least operations per subset
 // among those whose code stays within kElimOps instructions (compile time)
 // and whose tables within kElimPeak values, leaving at least 2^19 outer
@@ -859,14 +892,13 @@ static void emit_real_tail(std::ostringstream& o)
 // order 30 with 4 0.11, 0.013.  Below order 26 a walk takes 0.02 ms.
 int real_elim_columns(const double* b, int n)
 {
-    constexpr int kElimOps = 1000, kElimPeak = 128;
     if (n < 26) return 0;
     const std::vector<double> v(b, b + (size_t)n * n);
     int best = 0;
     double least = 1e300;
     for (int m = 3; m <= std::min(16, n - 20); ++m) {
         int ops = 0, peak = 0, outer = 0;
-        if (!Eliminator(v, n, m).run(ops, peak, nullptr, "") || ops > kElimOps || peak > kElimPeak) continue;
+        if (!Eliminator(v, n, m).run(ops, peak, kElimOps, kElimPeak)) continue;
         for (int r = 0; r < n; ++r) {
             bool in = false;
             for (int c = 0; c < m; ++c) in = in || b[(size_t)r * n + c] != 0.0;
@@ -892,7 +924,7 @@ static std::string emit_real_elim_kernel(const std::vector<double>& b, int n, bo
     }
     int ops = 0, peak = 0;
     std::string inner;
-    Eliminator(b, n, m).run(ops, peak, &inner, "            ");
+    Eliminator(b, n, m).run(ops, peak, kElimOps, kElimPeak, &inner, "            ");
     std::ostringstream o;
     o << "// generated: SpaRyser kernel for one " << n << "x" << n << " real matrix (FP64, "
       << (compensated ? "compensated" : "plain") << " sums, " << m << " inner columns summed out in " << ops
@@ -965,9 +997,9 @@ static std::string emit_real_elim_kernel(const std::vector<double>& b, int n, bo
     return o.str();
 }
 
-std::string emit_real_kernel(const std::vector<double>& b, int n, bool compensated, const std::string& name)
+std::string emit_real_kernel(const std::vector<double>& b, int n, bool compensated, const std::string& name, int elim)
 {
-    if (const int m = real_elim_columns(b.data(), n)) return emit_real_elim_kernel(b, n, compensated, name, m);
+    if (elim > 0) return emit_real_elim_kernel(b, n, compensated, name, elim);
     const int U = gen_unroll_bits_real(n);
     const RealLevels lv = real_levels(b, n);
     std::vector<double> x0(n);

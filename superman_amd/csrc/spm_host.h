@@ -122,7 +122,8 @@ void ut_order(const int64_t* a, int n, std::vector<int>& rowPerm, std::vector<in
 int codegen_compile_only(const std::string& src, const std::string& name, double* seconds, size_t* code_bytes);
 std::vector<int64_t> apply_perm(const int64_t* a, int n, const std::vector<int>& rp, const std::vector<int>& cp);
 std::string emit_int_kernel(const std::vector<int64_t>& b, int n, const std::string& name);
-std::string emit_real_kernel(const std::vector<double>& b, int n, bool compensated, const std::string& name);
+// elim: real_elim_columns of b.
+std::string emit_real_kernel(const std::vector<double>& b, int n, bool compensated, const std::string& name, int elim);
 int real_levels_count(const std::vector<double>& b, int n);
 uint64_t real_pattern_hash(const double* b, int n, int options, int precision);
 // log2 of a generated kernel's block length: real kernels by order, integer
