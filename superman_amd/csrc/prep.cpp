@@ -38,13 +38,14 @@ void dense_prepare(const double* a, int n, int w, double* planes, double* x0)
 namespace {
 
 // Whether sums of a row's entries are exact in FP64 (entries of few bits, such
-// as integers): then x has no rounding to lose.
-bool exact_sums(const double* a, int entries)
+// as integers): then x has no rounding to lose.  Each row by itself: rows of
+// different scales never meet in a sum.
+bool exact_sums(const double* r, int entries)
 {
     int top = -1, low = 1 << 20;  // in bits above 2^-1074
     for (int e = 0; e < entries; ++e) {
         uint64_t u;
-        std::memcpy(&u, a + e, 8);
+        std::memcpy(&u, r + e, 8);
         const int x = (int)((u >> 52) & 0x7ff);
         const uint64_t m = (u & ((uint64_t(1) << 52) - 1)) | (x ? uint64_t(1) << 52 : 0);
         if (m == 0) continue;
@@ -86,12 +87,12 @@ int pivot_column(const double* least, int n, Allowed allowed)
 //   - every column has a zero (or an entry 2^-60 of its row's largest), or
 //     the row bounds sum_j |a_ij| / |c_i| multiply past 2^900 (products near
 //     overflow);
-//   - the row sums are exact as they are (integers, say) and the quotients
-//     would not be: a column of powers of two is taken there, or none.
+//   - a row's sums are exact as they are (integers, say) and its quotients
+//     would not be: such rows need a power of two in the column.
 bool pair_prepare(const double* a, int n, double* out, PairScale* scale)
 {
     if (n < kPairMinN) return false;
-    const bool exact = exact_sums(a, n * n);
+    bool exact[kMaxN];
     double least[kMaxN];  // per column: the smallest |a_ij| / max_k |a_ik|
     std::fill(least, least + n, 1.0);
     for (int i = 0; i < n; ++i) {
@@ -99,11 +100,12 @@ bool pair_prepare(const double* a, int n, double* out, PairScale* scale)
         double top = 0.0;
         for (int j = 0; j < n; ++j) top = std::max(top, std::fabs(r[j]));
         if (top == 0.0) return false;
+        exact[i] = exact_sums(r, n);
         for (int j = 0; j < n; ++j) least[j] = std::min(least[j], std::fabs(r[j]) / top);
     }
     const int col = pivot_column(least, n, [&](int j) {
-        for (int i = 0; exact && i < n; ++i)
-            if (!power_of_two(a[(size_t)i * n + j])) return false;
+        for (int i = 0; i < n; ++i)
+            if (exact[i] && !power_of_two(a[(size_t)i * n + j])) return false;
         return true;
     });
     if (col < 0) return false;
@@ -145,12 +147,12 @@ bool pair_prepare(const double* a, int n, double* out, PairScale* scale)
 // so the sums, |term| bounds included, need no scaling.  Entries are rounded
 // once, from long double: with the factors rounded to double first (2 us less
 // at order 21) Haar orders 12 and 16 lost 1.2x against 64 bits.  The column
-// and the cases it is refused for are pair_prepare's; an exact matrix needs a
-// column of +-2^k, +-i 2^k.
+// and the cases it is refused for are pair_prepare's; an exact row needs +-2^k
+// or +-i 2^k in the column, an exact row n-2 needs it of all rows.
 bool pair_prepare_complex(const double* a, int n, double* out)
 {
     if (n < kPairMinN) return false;
-    const bool exact = exact_sums(a, 2 * n * n);
+    bool exact[kMaxComplexN];
     double least[kMaxComplexN];
     std::fill(least, least + n, 1.0);
     for (int i = 0; i < n; ++i) {
@@ -158,11 +160,13 @@ bool pair_prepare_complex(const double* a, int n, double* out)
         double top = 0.0;
         for (int e = 0; e < 2 * n; ++e) top = std::max(top, std::fabs(r[e]));
         if (top == 0.0) return false;
+        exact[i] = exact_sums(r, 2 * n);
         for (int j = 0; i + 2 < n && j < n; ++j)
             least[j] = std::min(least[j], std::max(std::fabs(r[2 * j]), std::fabs(r[2 * j + 1])) / top);
     }
     const int col = pivot_column(least, n, [&](int j) {
-        for (int i = 0; exact && i + 2 < n; ++i) {
+        for (int i = 0; i + 2 < n; ++i) {
+            if (!exact[i] && !exact[n - 2]) continue;
             const double re = a[(size_t)2 * (i * n + j)], im = a[(size_t)2 * (i * n + j) + 1];
             if (!(re == 0.0 ? power_of_two(im) : im == 0.0 && power_of_two(re))) return false;
         }
