@@ -88,8 +88,9 @@ struct Req {
 struct Slot {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    hipGraph_t graph[2] = {nullptr, nullptr};  // [organisation], captured when first used
+    hipGraphExec_t exec[2] = {nullptr, nullptr};
+    int own_int = 0;                // organisation of the current batch (kOwnIntWork)
     uint8_t* h_stage = nullptr;     // host-mapped, coherent: read by the upload kernel
     uint8_t* dh_stage = nullptr;    // its device address
     uint8_t* d_arena = nullptr;
@@ -146,6 +147,15 @@ bool dry(const spm_batch* b) { return b->cfg.executor == SPM_EXEC_DRYRUN; }
 // orders 10 to 25 took 1.04 instead of 0.95 ms; chunks half as long again (and
 // 2^8 real ones) spend more on chunk starts (400 requests 4.1 -> 4.4 ms).
 constexpr int kBatchFused = 1;
+// Above this much integer work (Req::work, about 2.5e-14 s each) a fused batch
+// leaves the integer items to their own kernel, launched behind the other
+// kinds'.  The complex walk's 195 VGPRs leave the fused kernel 2 waves per SIMD,
+// the integer kernel has 4 and walks 1.1 times as fast; but a launch more ends
+// in a tail more.  Fused / own: integers only, 300 of orders 22 to 25 7.52 / 6.84
+// ms, 20 of 26 to 28 5.64 / 5.10, 12 of 26 to 28 (1.3e11) 2.69 / 2.41, 300 of 14
+// to 20 1.59 / 1.64; 400 half real 8.78 / 8.53; a third of 24 of 26 to 28 (7.8e10)
+// 5.67 / 5.90; 256 mixed ones of 8 to 24 (5e9) 1.95 / 2.20.
+constexpr double kOwnIntWork = 1e11;
 constexpr int kBatchChunk[4] = {0, 10, 8, 9};  // [kind]
 // Chunk sizes of a request whose items at those sizes exceed the engine's.
 constexpr int kBatchChunkWide[4] = {0, 10, 9, 10};
@@ -292,10 +302,12 @@ void complete(spm_batch* b, Req* r, int status, const double* rec, double t_done
 
 void free_graph(Slot& s)
 {
-    if (s.exec) (void)hipGraphExecDestroy(s.exec);
-    if (s.graph) (void)hipGraphDestroy(s.graph);
-    s.exec = nullptr;
-    s.graph = nullptr;
+    for (int o = 0; o < 2; ++o) {
+        if (s.exec[o]) (void)hipGraphExecDestroy(s.exec[o]);
+        if (s.graph[o]) (void)hipGraphDestroy(s.graph[o]);
+        s.exec[o] = nullptr;
+        s.graph[o] = nullptr;
+    }
 }
 
 void free_slot(Slot& s)
@@ -333,12 +345,12 @@ hipError_t enqueue(spm_batch* b, Slot& s)
         e = hipLaunchKernel(batch_stage_kernel_ptr(), dim3(kStageBlocks), dim3(256), args, 0, s.stream);
         if (e != hipSuccess) return e;
     }
-    const int kinds[3] = {1, 2, 12};
-    for (int k = 0; k < (b->tune.fused ? 1 : 3); ++k) {
-        const int mask = b->tune.fused ? 15 : kinds[k];
-        const int q = b->tune.fused ? 0 : k + 1;
+    constexpr int kMask[4] = {15, 1, 2, 12};
+    constexpr int kLaunches[3][3] = {{0, -1, -1}, {0, 3, -1}, {1, 2, 3}};  // fused; fused and own integers; one a kind
+    for (int q : kLaunches[b->tune.fused ? s.own_int : 2]) {
+        if (q < 0) break;
         void* args[] = {&s.d_arena, &s.d_item, &s.d_counter, &done, &s.dh_res, &s.dh_flag};
-        e = hipLaunchKernel(batch_walk_kernel_ptr(mask), dim3(grid_for(b, q)), dim3(kDenseBlock), args, 0, s.stream);
+        e = hipLaunchKernel(batch_walk_kernel_ptr(kMask[q]), dim3(grid_for(b, q)), dim3(kDenseBlock), args, 0, s.stream);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -346,7 +358,6 @@ hipError_t enqueue(spm_batch* b, Slot& s)
 
 hipError_t capture(spm_batch* b, Slot& s)
 {
-    free_graph(s);
     hipError_t e = hipStreamBeginCapture(s.stream, hipStreamCaptureModeRelaxed);
     if (e != hipSuccess) return e;
     hipError_t e1 = enqueue(b, s);
@@ -357,8 +368,8 @@ hipError_t capture(spm_batch* b, Slot& s)
         return e1;
     }
     if (e != hipSuccess) return e;
-    s.graph = g;
-    return hipGraphInstantiate(&s.exec, g, nullptr, nullptr, 0);
+    s.graph[s.own_int] = g;
+    return hipGraphInstantiate(&s.exec[s.own_int], g, nullptr, nullptr, 0);
 }
 
 // Admission: FIFO with skip-ahead, within the slot's budgets.  Requests past
@@ -400,19 +411,21 @@ std::vector<Req*> admit(spm_batch* b, double now)
 
 // Writes header, descriptors, item table and data into the slot's staging
 // buffer; returns the bytes to upload.  Item order: shortest request first
-// (fused: over all kinds; per kind: grouped by kernel), so that small
+// (fused: over all kinds; else grouped by kernel), so that small
 // requests publish their results early; a large request's items are all of
 // one size, so the batch's tail is at most one item long.
 size_t stage(spm_batch* b, Slot& s, std::vector<Req*>& rs)
 {
-    if (b->tune.fused) {
-        std::stable_sort(rs.begin(), rs.end(), [](const Req* x, const Req* y) { return x->work < y->work; });
-    } else {
-        std::stable_sort(rs.begin(), rs.end(), [](const Req* x, const Req* y) {
-            const int gx = walk_group(x->dev_kind), gy = walk_group(y->dev_kind);
-            return gx != gy ? gx < gy : x->work < y->work;
-        });
-    }
+    double int_work = 0;
+    for (const Req* r : rs) int_work += walk_group(r->dev_kind) == kBatchInt ? r->work : 0;
+    s.own_int = b->tune.fused && int_work > kOwnIntWork ? 1 : 0;
+    auto group = [&](const Req* r) {  // launched after one another, in this order
+        const int g = walk_group(r->dev_kind);
+        return !b->tune.fused ? g : s.own_int && g == kBatchInt ? 1 : 0;
+    };
+    std::stable_sort(rs.begin(), rs.end(), [&](const Req* x, const Req* y) {
+        return group(x) != group(y) ? group(x) < group(y) : x->work < y->work;
+    });
     uint8_t* h = s.h_stage;
     BatchHeader hd;
     std::memset(&hd, 0, sizeof hd);
@@ -448,7 +461,7 @@ size_t stage(spm_batch* b, Slot& s, std::vector<Req*>& rs)
     }
     hd.items = item;
     hd.range_begin[0] = 0;
-    hd.range_end[0] = item;
+    hd.range_end[0] = s.own_int ? hd.range_begin[kBatchInt] : item;
     hd.bytes = data;
     std::memcpy(h, &hd, sizeof hd);
     return data;
@@ -487,8 +500,11 @@ int launch(spm_batch* b, Slot& s, std::vector<Req*>& rs, double now)
     hipError_t e = hipEventRecord(s.ev0, s.stream);
     if (e != hipSuccess) return fail(e, "hipEventRecord");
     if (b->cfg.use_graph) {
-        if (!s.exec && (e = capture(b, s)) != hipSuccess) return fail(e, "graph capture");
-        if ((e = hipGraphLaunch(s.exec, s.stream)) != hipSuccess) return fail(e, "hipGraphLaunch");
+        if (!s.exec[s.own_int] && (e = capture(b, s)) != hipSuccess) {
+            free_graph(s);
+            return fail(e, "graph capture");
+        }
+        if ((e = hipGraphLaunch(s.exec[s.own_int], s.stream)) != hipSuccess) return fail(e, "hipGraphLaunch");
     } else if ((e = enqueue(b, s)) != hipSuccess) {
         return fail(e, "kernel launch");
     }
