@@ -116,6 +116,7 @@ using namespace spm;
 struct spm_batch {
     spm_batch_config cfg{};
     spm_batch_tuning tune{};
+    bool chosen[4] = {false, false, false, false};  // [kind]: the caller set log2_chunk (geometry)
     int cus = 0;
     int max_wpc[4] = {0, 0, 0, 0};  // resident waves per CU: [0] fused, [kind] one-kind kernel
     size_t desc_off = 0, item_off = 0, data_off = 0, stage_bytes = 0;
@@ -157,7 +158,7 @@ constexpr int kBatchFused = 1;
 // 5.67 / 5.90; 256 mixed ones of 8 to 24 (5e9) 1.95 / 2.20.
 constexpr double kOwnIntWork = 1e11;
 constexpr int kBatchChunk[4] = {0, 10, 8, 9};  // [kind]
-// Chunk sizes of a request whose items at those sizes exceed the engine's.
+// The least chunk sizes of a request whose items at those exceed the engine's.
 constexpr int kBatchChunkWide[4] = {0, 10, 9, 10};
 // A request is split over up to 2^10 chunks (16 wavefronts) before its chunks
 // grow beyond 2^5 steps, since one wavefront's serial walk bounds a batch of
@@ -168,7 +169,9 @@ constexpr int kSplitSteps = 5;
 
 // Chunk size for a request: L >= 2 for the pipelined walks (n >= 3); n = 2
 // walks one 2-step chunk per lane (L = 1) and n = 1 its single subset.  It
-// follows from the request and the engine's configuration alone.
+// follows from the request and the engine's configuration alone.  A target
+// that the caller set is taken as it is; the engine's own (the default, or the
+// autotuner's) gives way to the split of small requests and to the item budget.
 void geometry(const spm_batch* b, Req* r)
 {
     const int B = r->n - 1;
@@ -178,10 +181,12 @@ void geometry(const spm_batch* b, Req* r)
     if (r->n == 1) L = 0;
     else if (r->n == 2) L = 1;
     else {
-        const int whole = std::max(2, std::min(target, B - 6));  // at least one full wavefront
-        L = std::min(whole, std::max(kSplitSteps, B - kSplitChunks));
-        if (items(L) > (uint64_t)b->cfg.max_items)
-            L = target == kBatchChunk[r->kind] ? std::max(2, std::min(kBatchChunkWide[r->kind], B - 6)) : whole;
+        auto whole = [&](int steps) { return std::max(2, std::min(steps, B - 6)); };  // at least one full wavefront
+        L = whole(target);
+        if (!b->chosen[r->kind]) {
+            L = std::min(L, std::max(kSplitSteps, B - kSplitChunks));
+            if (items(L) > (uint64_t)b->cfg.max_items) L = whole(std::max(target, kBatchChunkWide[r->kind]));
+        }
     }
     r->L = L;
     r->chunks = uint64_t(1) << (B - L);
@@ -873,7 +878,11 @@ extern "C" int spm_batch_set_tuning(spm_batch* b, const spm_batch_tuning* t)
 {
     if (!b || !t) return SPM_EINVAL;
     std::lock_guard<std::mutex> lk(b->mu);
-    return set_tuning_locked(b, t);
+    const spm_batch_tuning was = b->tune;
+    const int st = set_tuning_locked(b, t);
+    for (int k = 1; st == SPM_OK && k < 4; ++k)  // (a value written back as it was read is no choice)
+        if (t->log2_chunk[k] != was.log2_chunk[k]) b->chosen[k] = true;
+    return st;
 }
 
 extern "C" int spm_batch_run(spm_batch* b, int count, const spm_request* reqs, spm_result* out)
