@@ -73,7 +73,7 @@ typedef struct spm_result {
     double kernel_ms;     /* device time of the permanent kernels, by its clock */
     uint64_t subsets;     /* 2^(n-1) Gray-code subsets walked               */
     int32_t n;
-    int32_t launches;
+    int32_t launches;     /* kernels that formed the sum (without upload and result) */
 } spm_result;
 
 const char* spm_version(void);
@@ -205,7 +205,9 @@ int spm_plan_codegen_info(const spm_plan* plan, double* compile_seconds, int* ca
 int spm_plan_run(spm_plan* plan, void* stream, spm_result* out);
 int spm_plan_destroy(spm_plan* plan);
 /* Launch geometry of a plan: grid blocks, block threads, L (Gray steps per
- * chunk = 2^L), number of wave tasks. */
+ * chunk = 2^L), number of wave tasks.  Of a pruned integer plan, which walks
+ * no chunks: the node kernel's grid, L = 0, and the settings of the outermost
+ * columns that the search starts from. */
 int spm_plan_info(const spm_plan* plan, int* grid, int* block, int* log2_chunk, uint64_t* tasks);
 /* The Gray-walk geometry the dense kernels use for order n when
  * `resident_waves` wavefronts fit on the device: each lane walks 2^log2_chunk

@@ -969,6 +969,7 @@ static int int_run(spm_plan* p, hipStream_t st, spm_result* r)
         if (p->d_counter) {
             rc = prune_launch(p, tb, te, st);
             if (rc != SPM_OK) return rc;
+            launches += p->first_group - 1;  // the tables and the lists before the nodes
         } else if (p->kind == 4) {
             void* args[] = {&p->d_partial, &tb, &te, &p->chunks, &p->L, &acc};
             if (hipModuleLaunchKernel(p->fn, p->grid, 1, 1, kDenseBlock, 1, 1, 0, st, args, nullptr) != hipSuccess)
@@ -1018,7 +1019,7 @@ extern "C" int spm_plan_destroy(spm_plan* p)
 extern "C" int spm_plan_info(const spm_plan* p, int* grid, int* block, int* log2_chunk, uint64_t* tasks)
 {
     if (!p) return SPM_EINVAL;
-    if (grid) *grid = p->grid;
+    if (grid) *grid = p->kern2 ? p->grid2 : p->grid;  // pruned: the walk over the nodes
     if (block) *block = p->block;
     if (log2_chunk) *log2_chunk = p->L;
     if (tasks) *tasks = p->tasks;
