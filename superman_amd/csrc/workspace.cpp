@@ -4,7 +4,8 @@
 // pinned memory used to come from the runtime each time, 25-60 us of a call
 // that takes 10 us on the GPU.  Dropped workspaces wait here instead, at most
 // kIdleMax of them and kIdleBytes of device memory per device; whatever
-// exceeds that is freed.  A workspace belongs to one plan at a time, and a plan
+// exceeds that is freed, and all of them are when an allocation fails: a call
+// that fits the device without the pool fits it with the pool.  A workspace belongs to one plan at a time, and a plan
 // gives it back only after its last run's result has arrived, so no two
 // streams or threads ever share one.
 #include "workspace.h"
@@ -35,6 +36,36 @@ void release(Workspace* w)
     delete w;
 }
 
+Workspace* allocate(int device, size_t dev_bytes, size_t host_bytes)
+{
+    Workspace* w = new Workspace;
+    w->device = device;
+    w->dev_bytes = dev_bytes;
+    w->host_bytes = host_bytes;
+    if (hipMalloc((void**)&w->dev, dev_bytes) != hipSuccess ||
+        hipHostMalloc((void**)&w->host, host_bytes + sizeof(RunResult), hipHostMallocMapped | hipHostMallocCoherent) !=
+            hipSuccess ||
+        hipHostGetDevicePointer((void**)&w->host_dev, w->host, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        release(w);
+        return nullptr;
+    }
+    w->result_host = (RunResult*)(w->host + host_bytes);
+    w->result = (RunResult*)(w->host_dev + host_bytes);
+    w->result_host->flag = 0;
+    return w;
+}
+
+void release_idle()
+{
+    std::vector<Workspace*> drop;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        drop.swap(g_idle);
+    }
+    for (Workspace* w : drop) release(w);
+}
+
 size_t rounded(size_t bytes, size_t least)
 {
     size_t s = least;
@@ -58,23 +89,14 @@ int workspace_get(int device, size_t dev_bytes, size_t host_bytes, Workspace** o
             }
         }
     }
-    Workspace* w = new Workspace;
-    w->device = device;
-    w->dev_bytes = need;
-    w->host_bytes = hneed;
-    if (hipMalloc((void**)&w->dev, need) != hipSuccess ||
-        hipHostMalloc((void**)&w->host, hneed + sizeof(RunResult), hipHostMallocMapped | hipHostMallocCoherent) !=
-            hipSuccess ||
-        hipHostGetDevicePointer((void**)&w->host_dev, w->host, 0) != hipSuccess) {
-        (void)hipGetLastError();
-        release(w);
-        return SPM_ENOMEM;
+    Workspace* w = allocate(device, need, hneed);
+    if (!w) {
+        release_idle();
+        w = allocate(device, need, hneed);
     }
-    w->result_host = (RunResult*)(w->host + hneed);
-    w->result = (RunResult*)(w->host_dev + hneed);
-    w->result_host->flag = 0;
+    if (!w) w = allocate(device, (dev_bytes + 255) & ~size_t(255), (host_bytes + 255) & ~size_t(255));
     *out = w;
-    return SPM_OK;
+    return w ? SPM_OK : SPM_ENOMEM;
 }
 
 void workspace_put(Workspace* w, bool idle)
