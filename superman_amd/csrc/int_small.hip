@@ -27,7 +27,7 @@ int_small_kernel(const double* __restrict__ M,            // [2][N][N]: +2A, -2A
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint64_t wave = (uint64_t)blockIdx.x * (kDenseBlock / kWave) + (threadIdx.x / kWave);
     const uint64_t nwave = (uint64_t)gridDim.x * (kDenseBlock / kWave);
-    touch_lines<2 * N * N, kDenseBlock>(M, threadIdx.x);
+    if constexpr (real::kIntFpColdStart<N>) touch_lines<2 * N * N, kDenseBlock>(M, threadIdx.x);
     unsigned __int128 acc = 0;
     for (uint64_t task = task_begin + wave; task < task_end; task += nwave) {
         const uint64_t h = task * kWave + lane;

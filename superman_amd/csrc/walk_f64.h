@@ -328,8 +328,9 @@ struct F32ProdTerm {
 
 // One lane's chunk: the 2^L Gray steps starting at k = h 2^L over the walked
 // columns 0..NC-1 of M (column stride N), every term handed to `term`, which
-// folds FOLD steps at a time.
-template <int N, int U, class Term, int NC = N - 1, uint32_t FOLD = kFoldSteps>
+// folds FOLD steps at a time.  SKIP: columns that no lane of the wave starts
+// with are not read.
+template <int N, int U, class Term, int NC = N - 1, uint32_t FOLD = kFoldSteps, bool SKIP = true>
 __device__ __forceinline__ void walk_gray(const double* __restrict__ M,   // [2][N][N]: +A, -A
                                           const double* __restrict__ x0,  // x(empty set)
                                           uint64_t h, int L, Term& term)
@@ -348,15 +349,16 @@ __device__ __forceinline__ void walk_gray(const double* __restrict__ M,   // [2]
     // Columns >= L + 6 are set or not for the whole wave (its chunks are 64
     // neighbours): those that are not are not read (order 21 11.9 -> 10.9 us a
     // run, complex 24.5 -> 22.2 us).
-    const int shared = min(NC, L + 6);
+    const int shared = SKIP ? min(NC, L + 6) : NC;
     for (int j = (L > 0 ? L - 1 : 0); j < shared; ++j) {
         const double b = ((g0 >> j) & 1u) ? 1.0 : 0.0;
         const const_f64* __restrict__ col = step_column(M + j * N);
 #pragma unroll
         for (int r = 0; r < N; ++r) x[r] = __builtin_fma(b, col[r], x[r]);
     }
-    for (uint64_t left = wave_bits(g0) & ((uint64_t(1) << NC) - (uint64_t(1) << shared)); left != 0; left &= left - 1)
-        flip_const<N, false>(x, M + __builtin_ctzll(left) * N);
+    if constexpr (SKIP)
+        for (uint64_t left = wave_bits(g0) & ((uint64_t(1) << NC) - (uint64_t(1) << shared)); left != 0; left &= left - 1)
+            flip_const<N, false>(x, M + __builtin_ctzll(left) * N);
 
     const double lane_sign = (h & 1u) ? -1.0 : 1.0;  // direction of column L-1
     const uint32_t nblk = 1u << (L - U);

@@ -70,6 +70,14 @@ struct SmallIntTerm {
     __device__ __forceinline__ void fold() {}
 };
 
+// Up to order 31 the kernel touches the matrix first and a chunk start reads the
+// set columns only.  Past it chunk starts are a hundredth of the walk, and its
+// registers suffer from that: 187-205 VGPRs from order 33 on, 2 waves per SIMD,
+// instead of 120-153 and 4 or 3.  Half 0/1, with / without: order 32 7.34 / 7.15
+// ms, order 34 40.9 / 36.0, order 36 151.8 / 139.4.
+template <int N>
+constexpr bool kIntFpColdStart = N <= 31;
+
 // T mod 2^128 over one lane's chunk.  M = [2][N][N] doubles (+2A, -2A),
 // y0 = y(empty set) as doubles.
 template <int N>
@@ -77,7 +85,7 @@ __device__ __forceinline__ unsigned __int128 walk_intfp(const double* __restrict
                                                         uint64_t h, int L)
 {
     SmallIntTerm<N> term;
-    walk_gray<N, kDenseUnroll<N>>(M, y0, h, L, term);
+    walk_gray<N, kDenseUnroll<N>, SmallIntTerm<N>, N - 1, kFoldSteps, kIntFpColdStart<N>>(M, y0, h, L, term);
     return term.acc;
 }
 
