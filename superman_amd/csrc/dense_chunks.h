@@ -10,7 +10,8 @@ namespace spm {
 
 // The grid-strided task loop over one matrix's chunks and the block
 // reduction into per-block records, for the accumulation policy Term.
-template <int N, int U, class Term, int NC = N - 1, uint32_t FOLD = real::kFoldSteps>
+// COLD: the matrix is touched first and a chunk start reads the set columns only.
+template <int N, int U, class Term, int NC = N - 1, uint32_t FOLD = real::kFoldSteps, bool COLD = true>
 __device__ __forceinline__ void dense_chunks(const double* __restrict__ M, const double* __restrict__ x0,
                                              double* __restrict__ partial, uint64_t task_begin,
                                              uint64_t task_end, uint64_t num_chunks, int L, int accumulate)
@@ -21,13 +22,14 @@ __device__ __forceinline__ void dense_chunks(const double* __restrict__ M, const
     const uint64_t wave = (uint64_t)blockIdx.x * (kDenseBlock / kWave) + (threadIdx.x / kWave);
     const uint64_t nwave = (uint64_t)gridDim.x * (kDenseBlock / kWave);
 
-    touch_lines<(N + 1 + NC) * N, kDenseBlock>(M, threadIdx.x);  // M is column N - 1 - NC of the first plane
+    if constexpr (COLD)
+        touch_lines<(N + 1 + NC) * N, kDenseBlock>(M, threadIdx.x);  // M is column N - 1 - NC of the first plane
     double acc_hi = 0.0, acc_lo = 0.0, acc_abs = 0.0;
     for (uint64_t task = task_begin + wave; task < task_end; task += nwave) {
         const uint64_t h = task * kWave + lane;
         const bool active = h < num_chunks;  // lanes past the end walk a dummy chunk
         Term term;
-        real::walk_gray<N, U, Term, NC, FOLD>(M, x0, h, L, term);
+        real::walk_gray<N, U, Term, NC, FOLD, COLD>(M, x0, h, L, term);
         if (active) {
             if constexpr (COMP) {
                 dd_add(acc_hi, acc_lo, term.t_hi, term.t_lo);

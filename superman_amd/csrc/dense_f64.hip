@@ -20,7 +20,11 @@ dense_f64_kernel(const double* __restrict__ M,   // [2][N][N]: +A then -A, colum
                  uint64_t task_begin, uint64_t task_end, uint64_t num_chunks, int L,
                  int accumulate)
 {
-    dense_chunks<N, U, real::FpTerm<N, COMP>>(M, x0, partial, task_begin, task_end, num_chunks, L, accumulate);
+    // Past order 36 a run takes 140 ms and more, nothing of it cold, and the chunk
+    // starts that read set columns only can cost the steps' schedule: plain order
+    // 38 292.7 ms with them, 281.8 without (order 36 66.7 and 67.7).
+    dense_chunks<N, U, real::FpTerm<N, COMP>, N - 1, real::kFoldSteps, N <= 36>(M, x0, partial, task_begin, task_end,
+                                                                               num_chunks, L, accumulate);
 }
 
 // FP32-product variant for nonnegative, row-scaled matrices (same records
