@@ -340,9 +340,9 @@ typedef struct spm_batch_config {
 } spm_batch_config;
 
 typedef struct spm_batch_tuning {
-    int fused;              /* 1: one kernel walks every kind (batches with much
-                               integer work leave that to its own kernel, behind
-                               the other kinds); 0: one per kind                    */
+    int fused;              /* 1: one kernel walks every kind (batches of mostly
+                               integer work, if it is much, leave that to its own
+                               kernel, behind the other kinds); 0: one per kind     */
     int waves_per_cu;       /* persistent grid size (0 = all resident waves)        */
     int log2_chunk[4];      /* [kind]: target Gray steps per lane chunk (2^L).  A
                                value set other than the one read is taken as it is

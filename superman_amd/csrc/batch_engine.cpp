@@ -117,6 +117,7 @@ struct spm_batch {
     spm_batch_config cfg{};
     spm_batch_tuning tune{};
     bool chosen[4] = {false, false, false, false};  // [kind]: the caller set log2_chunk (geometry)
+    bool all_fused = false;  // no kernel of their own for the integers (autotuning on a mix's integer requests)
     int cus = 0;
     int max_wpc[4] = {0, 0, 0, 0};  // resident waves per CU: [0] fused, [kind] one-kind kernel
     size_t desc_off = 0, item_off = 0, data_off = 0, stage_bytes = 0;
@@ -148,14 +149,17 @@ bool dry(const spm_batch* b) { return b->cfg.executor == SPM_EXEC_DRYRUN; }
 // orders 10 to 25 took 1.04 instead of 0.95 ms; chunks half as long again (and
 // 2^8 real ones) spend more on chunk starts (400 requests 4.1 -> 4.4 ms).
 constexpr int kBatchFused = 1;
-// Above this much integer work (Req::work, about 2.5e-14 s each) a fused batch
-// leaves the integer items to their own kernel, launched behind the other
-// kinds'.  The complex walk's 195 VGPRs leave the fused kernel 2 waves per SIMD,
-// the integer kernel has 4 and walks 1.1 times as fast; but a launch more ends
-// in a tail more.  Fused / own: integers only, 300 of orders 22 to 25 7.52 / 6.84
-// ms, 20 of 26 to 28 5.64 / 5.10, 12 of 26 to 28 (1.3e11) 2.69 / 2.41, 300 of 14
-// to 20 1.59 / 1.64; 400 half real 8.78 / 8.53; a third of 24 of 26 to 28 (7.8e10)
-// 5.67 / 5.90; 256 mixed ones of 8 to 24 (5e9) 1.95 / 2.20.
+// With more than this much integer work (Req::work, about 2.5e-14 s each), and
+// more than half of its work integer, a fused batch leaves the integer items to
+// their own kernel, launched behind the other kinds'.  The complex walk's 195
+// VGPRs leave the fused kernel 2 waves per SIMD, the integer kernel has 4 and
+// walks 1.1 times as fast; but a launch more ends in a tail more, and small
+// integer requests wait for the other kinds.  Fused / own: integers only, 300 of
+// orders 22 to 25 7.52 / 6.84 ms, 20 of 26 to 28 5.64 / 5.10, 12 of 26 to 28
+// (1.3e11) 2.69 / 2.41, 300 of 14 to 20 (5e9) 1.59 / 1.64; 300 a quarter real
+// 7.35 / 6.88, half real 8.78 / 8.53, a quarter complex (65 % integer work) 9.12 /
+// 9.07, half complex (38 %) 10.2 / 10.6.  Orders 8 to 28, 20 % integer (23 %), at
+// the plain path's load: p99 1.82 / 1.98 ms.
 constexpr double kOwnIntWork = 1e11;
 constexpr int kBatchChunk[4] = {0, 10, 8, 9};  // [kind]
 // The least chunk sizes of a request whose items at those exceed the engine's.
@@ -421,9 +425,12 @@ std::vector<Req*> admit(spm_batch* b, double now)
 // one size, so the batch's tail is at most one item long.
 size_t stage(spm_batch* b, Slot& s, std::vector<Req*>& rs)
 {
-    double int_work = 0;
-    for (const Req* r : rs) int_work += walk_group(r->dev_kind) == kBatchInt ? r->work : 0;
-    s.own_int = b->tune.fused && int_work > kOwnIntWork ? 1 : 0;
+    double work = 0, int_work = 0;
+    for (const Req* r : rs) {
+        work += r->work;
+        int_work += walk_group(r->dev_kind) == kBatchInt ? r->work : 0;
+    }
+    s.own_int = b->tune.fused && !b->all_fused && int_work > kOwnIntWork && int_work > 0.5 * work ? 1 : 0;
     auto group = [&](const Req* r) {  // launched after one another, in this order
         const int g = walk_group(r->dev_kind);
         return !b->tune.fused ? g : s.own_int && g == kBatchInt ? 1 : 0;
@@ -963,6 +970,11 @@ extern "C" int spm_batch_autotune(spm_batch* b, int count, const spm_request* sa
         for (int i = 0; i < count; ++i)
             if (sample[i].kind == k) sub.push_back(sample[i]);
         if (sub.empty()) continue;
+        struct AllFused {
+            spm_batch* b;
+            ~AllFused() { b->all_fused = false; }
+        } scope{b};
+        b->all_fused = (int)sub.size() < count;
         // (L, seconds), the starting chunk first: it must run, the others
         // are dropped (1e300) when their launches fail
         std::vector<std::pair<int, double>> tried(1, {win.log2_chunk[k], 0.0});
