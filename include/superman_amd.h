@@ -344,11 +344,12 @@ typedef struct spm_batch_tuning {
                                integer work, if it is much, leave that to its own
                                kernel, behind the other kinds); 0: one per kind     */
     int waves_per_cu;       /* persistent grid size (0 = all resident waves)        */
-    int log2_chunk[4];      /* [kind]: target Gray steps per lane chunk (2^L).  A
-                               value set other than the one read is taken as it is
-                               from then on.  Under the engine's own (the default,
-                               the autotuner's) small requests walk shorter chunks,
-                               and those that would exceed max_items longer ones    */
+    int log2_chunk[4];      /* [kind]: Gray steps per lane chunk (2^L), an upper
+                               limit: requests up to order 20 or so are split
+                               further.  A request that then exceeds max_items
+                               walks longer chunks, under a value that was set
+                               (other than the one read) of that size, and is
+                               refused when those exceed max_items too             */
 } spm_batch_tuning;
 
 typedef struct spm_request {

@@ -173,9 +173,12 @@ constexpr int kSplitSteps = 5;
 
 // Chunk size for a request: L >= 2 for the pipelined walks (n >= 3); n = 2
 // walks one 2-step chunk per lane (L = 1) and n = 1 its single subset.  It
-// follows from the request and the engine's configuration alone.  A target
-// that the caller set is taken as it is; the engine's own (the default, or the
-// autotuner's) gives way to the split of small requests and to the item budget.
+// follows from the request and the engine's configuration alone.  The target is
+// an upper limit: small requests are split further, by whatever target (with the
+// autotuner's sizes set on a second engine and taken as they are, the serving mix
+// at the plain path's load had a p99 of 1.95 instead of 1.82 ms).  The item budget
+// lengthens chunks of the engine's own sizes only: one that the caller set is
+// refused there.
 void geometry(const spm_batch* b, Req* r)
 {
     const int B = r->n - 1;
@@ -186,11 +189,9 @@ void geometry(const spm_batch* b, Req* r)
     else if (r->n == 2) L = 1;
     else {
         auto whole = [&](int steps) { return std::max(2, std::min(steps, B - 6)); };  // at least one full wavefront
-        L = whole(target);
-        if (!b->chosen[r->kind]) {
-            L = std::min(L, std::max(kSplitSteps, B - kSplitChunks));
-            if (items(L) > (uint64_t)b->cfg.max_items) L = whole(std::max(target, kBatchChunkWide[r->kind]));
-        }
+        L = std::min(whole(target), std::max(kSplitSteps, B - kSplitChunks));
+        if (items(L) > (uint64_t)b->cfg.max_items)
+            L = whole(b->chosen[r->kind] ? target : std::max(target, kBatchChunkWide[r->kind]));
     }
     r->L = L;
     r->chunks = uint64_t(1) << (B - L);

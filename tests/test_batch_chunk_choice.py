@@ -1,5 +1,5 @@
-"""A chunk size that the caller sets is taken as it is; the engine's own gives
-way to the split of small requests and to the item budget."""
+"""A chunk size that the caller sets is an upper limit, and the one that counts
+for the item budget; the engine's own also gives way to that."""
 import numpy as np
 
 from superman_amd import _lib
@@ -18,21 +18,26 @@ def batches(eng, kind, n, count):
 
 
 def test_chunk_size_of_the_caller():
-    # order 20 complex: 2^19 subsets; chunks of 2^11 are 4 items of 64, of 2^7
-    # 64 items; the engine's own split of such a request takes 16
+    # order 20 complex, 2^19 subsets: the engine's 2^8 steps are 32 items of 64
+    # chunks, more than the budget, and give way to 2^9, the split's limit
     with BatchEngine(dry_run=True, max_items=16, slots=1) as eng:
-        assert batches(eng, "complex", 20, 8) == 8
+        assert batches(eng, "complex", 20, 4) == 4
         t = eng.tuning
         t.waves_per_cu = 8
         eng.tuning = t  # the chunk sizes written back as they were read
-        assert batches(eng, "complex", 20, 8) == 8
-        t.log2_chunk["complex"] = 11
+        assert batches(eng, "complex", 20, 4) == 4
+        for steps, st in ((11, 0), (9, 0), (7, _lib.SPM_ENOMEM), (8, _lib.SPM_ENOMEM)):
+            t.log2_chunk["complex"] = steps  # (8 is the default's value, now set)
+            eng.tuning = t
+            assert eng.try_submit("complex", make("complex", 20))[0] == st, steps
+            while eng.poll() or eng.progress():
+                pass
+        assert batches(eng, "real", 20, 4) == 4  # the other kinds keep the engine's
+    with BatchEngine(dry_run=True, max_items=64, slots=1) as eng:
+        t = eng.tuning
+        t.log2_chunk["complex"] = 13  # split to 2^9 steps all the same: 4 requests a batch
         eng.tuning = t
         assert batches(eng, "complex", 20, 8) == 2
-        t.log2_chunk["complex"] = 7
+        t.log2_chunk["complex"] = 7  # as short as it is set: one request a batch
         eng.tuning = t
-        assert eng.try_submit("complex", make("complex", 20))[0] == _lib.SPM_ENOMEM
-        assert batches(eng, "real", 20, 8) == 8  # the other kinds keep the engine's
-        t.log2_chunk["complex"] = 8  # the default's value, set: 32 items
-        eng.tuning = t
-        assert eng.try_submit("complex", make("complex", 20))[0] == _lib.SPM_ENOMEM
+        assert batches(eng, "complex", 20, 8) == 8
