@@ -158,8 +158,7 @@ constexpr int kBatchFused = 1;
 // orders 22 to 25 7.52 / 6.84 ms, 20 of 26 to 28 5.64 / 5.10, 12 of 26 to 28
 // (1.3e11) 2.69 / 2.41, 300 of 14 to 20 (5e9) 1.59 / 1.64; 300 a quarter real
 // 7.35 / 6.88, half real 8.78 / 8.53, a quarter complex (65 % integer work) 9.12 /
-// 9.07, half complex (38 %) 10.2 / 10.6.  Orders 8 to 28, 20 % integer (23 %), at
-// the plain path's load: p99 1.82 / 1.98 ms.
+// 9.07, half complex (38 %) 10.2 / 10.6, a quarter integer (29 %) 9.9 / 10.3.
 constexpr double kOwnIntWork = 1e11;
 constexpr int kBatchChunk[4] = {0, 10, 8, 9};  // [kind]
 // The least chunk sizes of a request whose items at those exceed the engine's.
@@ -176,7 +175,7 @@ constexpr int kSplitSteps = 5;
 // follows from the request and the engine's configuration alone.  The target is
 // an upper limit: small requests are split further, by whatever target (with the
 // autotuner's sizes set on a second engine and taken as they are, the serving mix
-// at the plain path's load had a p99 of 1.95 instead of 1.82 ms).  The item budget
+// at the plain path's load had a p99 of 1.95 instead of 1.86 ms).  The item budget
 // lengthens chunks of the engine's own sizes only: one that the caller set is
 // refused there.
 void geometry(const spm_batch* b, Req* r)

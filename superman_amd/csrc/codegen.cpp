@@ -637,6 +637,10 @@ void emit_real_term(std::ostringstream& o, const RealLevels& lv, bool negative, 
 // about 600 operations, 0.3 per subset against 9 for the walk.  The same
 // tables of absolute values, added instead of subtracted, give sum |term|;
 // a product of rows alone shares its value (|ab| = |a||b| as rounded).
+// E is formed in FP64 under either precision (compensated sums begin with the
+// outer steps): it has far fewer roundings than the 2^m terms it replaces, and
+// against 80-bit values the results of 88 matrices (orders 26 to 38, 3 to 7
+// entries per row) are off by 0.2 of what the walk's are, geometric mean.
 // ---------------------------------------------------------------------------
 struct Factor {
     std::vector<int> scope;  // columns, ascending; entry i has column scope[k] set when bit k of i is
@@ -886,10 +890,13 @@ constexpr int kElimOps = 1000, kElimPeak = 128;
 // settings to share out.  0: walk.  The kernels take up to 512 VGPRs, one
 // wave per SIMD: straight-line code has its own parallelism, and at two
 // waves (256 VGPRs) the larger ones spill (order 38, 7 per row 6.0 -> 7.4 ms,
-// at three 20 ms).  Kernel ms of the walk and at 700 operations with 64
-// values, then 1200 with 128, N(0,1) entries: order 36 with 5 per row 8.1,
-// 0.39, 0.32; order 38 with 7 42, 6.0, 2.7; order 40 with 8 215, 55.7, 53.9;
-// order 30 with 4 0.11, 0.013.  Below order 26 a walk takes 0.02 ms.
+// at three 20 ms).  Kernel ms of the walk and at limits of 700 operations with
+// 64 values, then 1000 with 128, three N(0,1) matrices each: order 30 with 7 per
+// row 0.22-0.24, 0.04-0.09, 0.03-0.06; order 36 with 5 6.5-8.5, 0.06-0.26,
+// 0.03-0.18; order 38 with 7 36-39, 2.1-9.5, 2.1-4.3; order 40 with 8 175-191,
+// 40-67, 36-57 (1200 operations: the same but for one matrix).  A plan of such
+// a kernel takes 0.24-0.37 s, of a walk 0.25-0.33.  Below order 26 a walk takes
+// 0.02 ms.
 int real_elim_columns(const double* b, int n)
 {
     if (n < 26) return 0;

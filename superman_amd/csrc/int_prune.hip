@@ -5,7 +5,8 @@
 // What bounds it: VALU issue on the surviving nodes (about 5 instructions
 // per testable row and node of 4096 subsets) and terms (at order 30 about 105
 // instructions per 64 terms and 9 for each round of the queue); no memory but
-// the tables (10 to 60 KB, once per block).  Half 0/1 order 30: 226 us.
+// the tables (10 to 60 KB, once per block).  Half 0/1 order 30, a run: 247 to 312
+// us over four matrices with 15 to 18 even rows.
 #include "walk_prune.h"
 
 namespace spm {
